@@ -32,11 +32,13 @@
 
 #include <cfloat>
 #include <climits>
+#include <vector>
 
 #include "dev_util.h"
 #include "kernels_gpu.h"
 #include "launch.h"
 #include "matmul_mfma.h"
+#include "matmul_small.h"
 #include "quant_dev.h"
 
 namespace rpg {
@@ -1126,10 +1128,8 @@ void LaunchByShape(const char* name, const uint8_t* w, int64_t rows, int64_t row
 
 }  // namespace
 
-// Token counts from which the matrix-core GEMM replaces the tiled kernel
-// (measured on Qwen3-1.7B matrices: at 16 tokens 26 us vs 50 us for 6144 x 2048
-// Q4_K, 362 us vs 622 us for the 151936-row lm_head, but 22 us vs 19 us for
-// 2048 x 2048; from 32 tokens it wins for every shape).
+// Token counts from which the matrix-core GEMM replaces the tiled kernel where the
+// small-batch kernel (below) does not take the call.
 constexpr int64_t kMfmaMinTokens = 32;
 constexpr int64_t kMfmaMinTokensWide = 16;  // matrices of at least kMfmaWideRows rows
 constexpr int64_t kMfmaWideRows = 4096;
@@ -1143,6 +1143,25 @@ bool MfmaEligible(uint32_t type, const uint8_t* w_dev, const float* x_dev, int64
   const bool enough = n_tokens >= kMfmaMinTokens || (n_tokens >= kMfmaMinTokensWide && rows >= kMfmaWideRows);
   return (type == kGgmlQ4_K || type == kGgmlQ6_K) && enough && Aligned(x_dev, 16) && cols % kQK_K == 0 &&
          Aligned(w_dev, type == kGgmlQ4_K ? 16 : 2) && cols / kQK_K <= 0x7FFFFFFF;
+}
+
+}  // namespace
+
+namespace {
+
+// The small-batch kernel takes Q4_K / Q6_K matrices under the same alignment
+// rules, up to kSmallMaxTokens tokens (from there on the decoded-planes GEMM) and
+// where it is the faster one.
+constexpr int64_t kSmallMaxTokens = 511;
+SmallMat SmallOf(uint32_t type, const uint8_t* w_dev, int64_t rows, float* out) {
+  return SmallMat{w_dev, out, rows, type == kGgmlQ6_K};
+}
+bool SmallEligible(uint32_t type, const uint8_t* w_dev, const float* x_dev, int64_t rows, int64_t cols,
+                   int64_t n_tokens) {
+  return (type == kGgmlQ4_K || type == kGgmlQ6_K) && n_tokens >= 2 && n_tokens <= kSmallMaxTokens &&
+         Aligned(x_dev, 16) && cols % kQK_K == 0 && Aligned(w_dev, type == kGgmlQ4_K ? 16 : 2) && rows <= INT32_MAX - 16 &&
+         cols <= INT32_MAX &&
+         MatMulSmallWins(SmallOf(type, w_dev, rows, nullptr), static_cast<int32_t>(cols / kQK_K), n_tokens);
 }
 
 }  // namespace
@@ -1173,6 +1192,11 @@ void GpuMatMulQuantRaw(uint32_t type, const uint8_t* w_dev, int64_t rows, int64_
   const bool x_ok = Aligned(x_dev, 16) && cols % 4 == 0;
   const int64_t nb = cols / kQK_K;
   const bool generic = g_force_generic.load();
+  if (!generic && SmallEligible(type, w_dev, x_dev, rows, cols, n_tokens)) {
+    const SmallMat m = SmallOf(type, w_dev, rows, out_dev);
+    LaunchMatMulSmall(&m, 1, static_cast<int32_t>(nb), x_dev, n_tokens);
+    return;
+  }
   if (!generic && MfmaEligible(type, w_dev, x_dev, rows, cols, n_tokens)) {
     LaunchMatMulMfma(type, w_dev, rows, row_bytes, static_cast<int32_t>(nb), x_dev, cols, n_tokens, out_dev);
     return;
@@ -1349,6 +1373,27 @@ void GpuMatMulQuantGroup(const GpuTensor* const* ws, int32_t n_mats, const float
     for (int32_t i = 0; i < n_mats; ++i) GpuMatMulQuant(*ws[i], x_dev, n_tokens, outs[i]);
     return;
   }
+  // A few tokens: the matrices share launches. The others of the group follow as
+  // a group of their own.
+  std::vector<SmallMat> small;
+  std::vector<const GpuTensor*> rest;
+  std::vector<float*> rest_outs;
+  for (int32_t i = 0; i < n_mats; ++i) {
+    const uint8_t* w = static_cast<const uint8_t*>(ws[i]->buf.data());
+    if (SmallEligible(ws[i]->type, w, x_dev, ws[i]->rows, cols, n_tokens)) {
+      small.push_back(SmallOf(ws[i]->type, w, ws[i]->rows, outs[i]));
+    } else {
+      rest.push_back(ws[i]);
+      rest_outs.push_back(outs[i]);
+    }
+  }
+  if (!small.empty()) {
+    LaunchMatMulSmall(small.data(), static_cast<int32_t>(small.size()), static_cast<int32_t>(cols / kQK_K), x_dev, n_tokens);
+    if (rest.empty()) return;
+    ws = rest.data();
+    outs = rest_outs.data();
+    n_mats = static_cast<int32_t>(rest.size());
+  }
   // Prefill: the activations are split once for all the matrices (each output
   // bit-identical to its own GpuMatMulQuant call, which splits the same way).
   bool mfma = true;
@@ -1380,12 +1425,23 @@ void GpuMatMulQuantSwiGLU(const GpuTensor& w_gate, const GpuTensor& w_up, const 
             static_cast<long long>(w_gate.cols), static_cast<long long>(w_up.rows), static_cast<long long>(w_up.cols));
   RPG_CHECK(n_tokens > 0, "matmul: no tokens (n_tokens <= 0)");
   RPG_CHECK(x_dev != nullptr && gate_dev != nullptr && up_dev != nullptr, "GpuMatMulQuantSwiGLU got a null pointer");
+  const GpuTensor* mats[2] = {&w_gate, &w_up};
+  float* outs[2] = {gate_dev, up_dev};
   if (!g_force_generic.load() && SwiGLUDecodeEligible(w_gate, w_up, x_dev, n_tokens)) {
     DecodeSwiGLU(w_gate, w_up, x_dev, gate_dev, nullptr);
     return;
   }
-  const GpuTensor* mats[2] = {&w_gate, &w_up};
-  float* outs[2] = {gate_dev, up_dev};
+  if (!g_force_generic.load() && w_gate.type == w_up.type &&
+      SmallEligible(w_gate.type, static_cast<const uint8_t*>(w_gate.buf.data()), x_dev, w_gate.rows, w_gate.cols,
+                    n_tokens) &&
+      SmallEligible(w_up.type, static_cast<const uint8_t*>(w_up.buf.data()), x_dev, w_up.rows, w_up.cols, n_tokens)) {
+    CheckGroup(mats, 2, outs);
+    LaunchMatMulSmallSwiGLU(
+        SmallOf(w_gate.type, static_cast<const uint8_t*>(w_gate.buf.data()), w_gate.rows, gate_dev),
+        SmallOf(w_up.type, static_cast<const uint8_t*>(w_up.buf.data()), w_up.rows, nullptr),
+        static_cast<int32_t>(w_gate.cols / kQK_K), x_dev, n_tokens);
+    return;
+  }
   GpuMatMulQuantGroup(mats, 2, x_dev, n_tokens, outs);
   GpuSiluMulInPlace(gate_dev, up_dev, n_tokens * w_gate.rows);
 }

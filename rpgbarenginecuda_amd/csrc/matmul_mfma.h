@@ -37,6 +37,12 @@ void LaunchMatMulMfmaSplit(uint32_t type, const uint8_t* w, int64_t rows, int64_
 void LaunchMatMulMfma(uint32_t type, const uint8_t* w, int64_t rows, int64_t row_bytes, int32_t nb, const float* x,
                       int64_t cols, int64_t n_tokens, float* out);
 
+// A library-owned buffer of at least `bytes` for the partial results of K slices
+// (valid until the next split launch on the engine stream), and the launch that
+// sums them: out[e] = sum over z < splits of partial[z elems + e], in that order.
+float* SplitPartials(size_t bytes);
+void LaunchSplitReduce(const float* partial, int64_t elems, int32_t splits, float* out);
+
 }  // namespace rpg
 
 #endif  // RPG_AMD_MATMUL_MFMA_H_

@@ -1,0 +1,122 @@
+"""The small-batch quantised matmul (2 tokens to a medium prompt): every workgroup shape
+at the edges of its tiles, against the float64 oracle within the fp32 summation
+bound of tests/test_gpu_matmul.py, and against itself where the bits must agree."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import synth
+from test_gpu_matmul import check, dev, factored_magnitude, host
+
+pytestmark = pytest.mark.gpu
+
+Q4, Q6 = 12, 14
+
+SHAPES = [
+    # (type, rows, cols, tokens)
+    (Q4, 1, 256, 5), (Q6, 1, 256, 6),            # one row, one block
+    (Q4, 17, 768, 16), (Q6, 15, 768, 17),        # ragged row tile, odd blocks, one token over a tile
+    (Q6, 300, 2048, 31), (Q4, 300, 2048, 33),    # both sides of the slices' limit
+    (Q4, 2049, 2048, 65), (Q6, 2049, 2048, 97),  # ragged rows and token tiles, several tiles per workgroup
+    (Q4, 65, 2304, 9), (Q6, 65, 2560, 10),       # 9 and 10 blocks
+    (Q4, 1000, 2816, 8), (Q6, 1000, 2816, 40),   # 11 blocks: walked by a workgroup, in slices of unequal length
+    (Q6, 500, 9728, 30), (Q4, 500, 9728, 36),    # 38 blocks likewise
+    (Q6, 20000, 2048, 17), (Q4, 20000, 512, 21),  # many tiles
+]
+
+
+@pytest.mark.parametrize("t,rows,cols,n", SHAPES)
+def test_small_matmul_vs_f64(gpu, ora, t, rows, cols, n):
+    import torch
+
+    rng = np.random.default_rng(rows + cols + n + t)
+    w = synth.quant_table(rng, t, rows, cols)
+    x = rng.normal(0, 1, (n, cols)).astype(np.float32)
+    x[n // 2] *= 1e-20  # tokens of very different size keep their own scale
+    x[:, cols // 2] *= 1e3
+    out = torch.full((n + 1, rows), np.nan, dtype=torch.float32, device="cuda")
+    gpu.GpuMatMulQuant(gpu.GpuTensor(dev(w), t, rows, cols), dev(x), n, out[:n])
+    exact, absdot = ora.matmul_quant_f64(t, w, rows, cols, x)
+    check(host(out[:n]), exact, absdot, cols, factored_magnitude(ora, t, w, rows, cols, x))
+    assert torch.isnan(out[n]).all(), "wrote past the last token"
+
+
+@pytest.mark.parametrize("off", [2, 6, 14])
+def test_small_matmul_unaligned_q6k(gpu, off):
+    """A Q6_K matrix at any even address gives the bits of the aligned one."""
+    import torch
+
+    rows, cols, n = 130, 2560, 21
+    rng = np.random.default_rng(off)
+    w = dev(synth.quant_table(rng, Q6, rows, cols))
+    moved = torch.zeros(w.numel() + 64, dtype=torch.uint8, device="cuda")
+    moved[off:off + w.numel()] = w
+    x = dev(rng.normal(0, 1, (n, cols)).astype(np.float32))
+    outs = [torch.empty((n, rows), device="cuda") for _ in range(2)]
+    gpu.GpuMatMulQuant(gpu.GpuTensor(w, Q6, rows, cols), x, n, outs[0])
+    gpu.GpuMatMulQuant(gpu.GpuTensor(moved[off:off + w.numel()], Q6, rows, cols), x, n, outs[1])
+    assert torch.equal(*outs)
+
+
+@pytest.mark.parametrize("cols,n", [(2048, 21), (2048, 40), (2048, 200), (2560, 21), (2560, 70), (6144, 20), (6144, 50)])
+def test_small_group_and_swiglu_equal_separate_calls(gpu, cols, n):
+    """Matrices of both types and of sizes that prefer different shapes, each bit-identical to its own call;
+    gate / up likewise to the two products followed by SwiGLU."""
+    import torch
+
+    rng = np.random.default_rng(cols + n)
+    x = dev(rng.normal(0, 1, (n, cols)).astype(np.float32))
+    ws = [gpu.GpuTensor(dev(synth.quant_table(rng, t, r, cols)), t, r, cols)
+          for t, r in ((Q4, 2048), (Q4, 129), (Q6, 1024), (Q4, 9728), (Q4, 9728))]
+    alone = [torch.empty((n, w.rows), device="cuda") for w in ws]
+    for w, o in zip(ws, alone):
+        gpu.GpuMatMulQuant(w, x, n, o)
+    outs = [torch.empty_like(o) for o in alone]
+    gpu.GpuMatMulQuantGroup(ws, x, n, outs)
+    for w, a, o in zip(ws, alone, outs):
+        assert torch.equal(a, o), (w.type, w.rows)
+    gate, up = torch.empty_like(alone[3]), torch.empty_like(alone[4])
+    gpu.GpuMatMulQuantSwiGLU(ws[3], ws[4], x, n, gate, up)
+    gpu.GpuSiluMulInPlace(alone[3], alone[4], n * 9728)
+    assert torch.equal(gate, alone[3])
+
+
+@pytest.mark.parametrize("t", [Q4, Q6])
+@pytest.mark.parametrize("cols,n", [(2048, 40), (6144, 24), (6144, 48)])
+def test_small_one_hot_selects_columns(gpu, ora, t, cols, n):
+    """A single activation 1 gives the dequantised weight, bit for bit."""
+    import torch
+
+    rows = 40
+    rng = np.random.default_rng(t + cols + n)
+    w = synth.quant_table(rng, t, rows, cols)
+    picks = rng.permutation(cols)[:n]
+    x = np.zeros((n, cols), np.float32)
+    x[np.arange(n), picks] = 1.0
+    out = torch.empty((n, rows), device="cuda")
+    gpu.GpuMatMulQuant(gpu.GpuTensor(dev(w), t, rows, cols), dev(x), n, out)
+    want = ora.dequantize_row(t, w, rows * cols).reshape(rows, cols)[:, picks].T
+    assert np.array_equal(host(out), want)
+
+
+def test_small_matmul_captures_without_a_first_run(gpu):
+    """Below 32 tokens a call needs no buffer of the library, also for a long K."""
+    import torch
+
+    rows, cols, n = 64, 16384, 7
+    rng = np.random.default_rng(5)
+    w = gpu.GpuTensor(dev(synth.quant_table(rng, Q4, rows, cols)), Q4, rows, cols)
+    x = dev(rng.normal(0, 1, (n, cols)).astype(np.float32))
+    out, eager = torch.empty((n, rows), device="cuda"), torch.empty((n, rows), device="cuda")
+    st, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    st.wait_stream(torch.cuda.current_stream())
+    with gpu.ScopedEngineStream(st), torch.cuda.graph(g, stream=st):
+        gpu.GpuMatMulQuant(w, x, n, out)
+    for scale in (1.0, -2.0):
+        x *= scale
+        out.fill_(float("nan"))
+        g.replay()
+        gpu.GpuMatMulQuant(w, x, n, eager)
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
