@@ -877,7 +877,10 @@ __device__ __forceinline__ F16x4 VTr(const _Float16* lds_ptr) {
 // the packed pair: the same bits as converting h back, subtracting and
 // converting, in one instruction instead of three. (Written out because the
 // compiler folds a multiply by -1 into a subtraction and then needs the
-// conversions.)
+// conversions.) The compiler does not see a vector ALU write in such a block, so
+// SplitPair puts the wait states itself that have to lie between the last write
+// and a matrix instruction that reads it; without them a schedule that multiplies
+// at once reads the registers' old contents.
 __device__ __forceinline__ uint32_t RemainderPair(uint32_t hpair, float x0, float x1) {
   uint32_t d;
   asm("v_fma_mixlo_f16 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]\n\t"
@@ -894,6 +897,7 @@ __device__ __forceinline__ void SplitPair(const float (&x)[8], F16x8* h, F16x8* 
   U32x4v lw;
 #pragma unroll
   for (int k = 0; k < 4; ++k) lw[k] = RemainderPair(hw[k], x[2 * k], x[2 * k + 1]);
+  asm("s_nop 1" : "+v"(lw));
   *l = __builtin_bit_cast(F16x8, lw);
 }
 
@@ -993,7 +997,14 @@ __global__ __launch_bounds__(256, 2) void AttnPrefillMfmaKernel(
 #pragma unroll
   for (int s = 0; s < 8; ++s) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) qv[s][j] *= qmul;
+    for (int j = 0; j < 8; ++j) {
+      qv[s][j] *= qmul;
+      // the rounded product, and not the exact one: given the choice the compiler
+      // rounds q qmul to fp16 in one step for one use and in two for another, and
+      // where they differ the remainder belongs to another first term (one row in
+      // 300 was off by 1e-4 relative)
+      asm("" : "+v"(qv[s][j]));
+    }
     qb[0][s] = SplitTerm(qv[s]);
     qb[1][s] = SplitTerm(qv[s]);
   }
