@@ -15,7 +15,9 @@
 //     when the max grows;
 //   * the no-cache path (GpuCausalAttention, fp32 k / v rows of the segment)
 //     runs the per-query-head kernel on fp32 rows;
-//   * decode and short prefills with a GQA group of 1, 2 or 4 use one wave per
+//   * turns of 2 to 63 tokens over a long cache run on the matrix cores, a workgroup
+//     per (32 tokens, query head) over all of the keys (AttnTurnKernel);
+//   * decode and other short prefills with a GQA group of 1, 2 or 4 use one wave per
 //     (token, kv head, chunk) for the whole group (AttnDecodeGroupKernel), other
 //     shapes one wave per query head (AttnChunkKernel);
 //   * prefill (many (t, h) pairs) uses a single chunk per pair and writes the
@@ -854,12 +856,10 @@ constexpr int kFaTokens = 128;    // tokens (of one head) per workgroup
 constexpr int kFaKeys = 64;       // keys per LDS block
 constexpr float kFaLazyLog2 = 8;  // the running max moves when a block's max exceeds it by more (log2 units)
 constexpr int kFaOrderMax = 1024; // (token tile, key chunk) pairs an ordered launch can list
-constexpr int kFaKStride = 136;   // halves per K row in LDS (128 + 8: conflict-free 16-byte reads)
 constexpr int kFaCounterStride = 16;       // uint32 slots between two (tile, head) arrival counters (64 bytes)
 constexpr int64_t kFaCounterSlots = 8192;  // (tile, head) counters per half (allocating / no-allocation)
 constexpr int kFaFusedMaxChunks = 4;       // key chunks the fused merge takes (more: a separate merge launch)
 constexpr int64_t kFaPartBlock = kFaTokens * (kD + 2);  // fused-merge partial floats per (tile, head, chunk)
-constexpr int kFaVStride = 160;   // halves per V row in LDS (128 + 32: conflict-free transposing reads)
 
 // ds_read_b64_tr_b16: in each 16-lane group, lane j receives element j % 4 of
 // the 8 bytes addressed by lanes j / 4, 4 + j / 4, 8 + j / 4, 12 + j / 4.
@@ -871,33 +871,44 @@ __device__ __forceinline__ F16x4 VTr(const _Float16* lds_ptr) {
   return __builtin_bit_cast(F16x4, v);
 }
 
+// 16 bytes per lane from global memory to LDS: lane i's at base + 16 i. The caller
+// waits (vmcnt) before it reads them.
+__device__ __forceinline__ void LoadToLds(const uint16_t* from, _Float16* base) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(from),
+                                   (__attribute__((address_space(3))) void*)(base), 16, 0, 0);
+}
+
 // x as two fp16 terms, *h = fp16(x) and *l = fp16(x - h) (the difference is
 // exact in fp32). Each remainder is one mixed-precision FMA, h * -1 + x with h
 // read as fp16 and the exact result rounded straight to fp16 into one half of
 // the packed pair: the same bits as converting h back, subtracting and
 // converting, in one instruction instead of three. (Written out because the
 // compiler folds a multiply by -1 into a subtraction and then needs the
-// conversions.) The compiler does not see a vector ALU write in such a block, so
-// SplitPair puts the wait states itself that have to lie between the last write
-// and a matrix instruction that reads it; without them a schedule that multiplies
-// at once reads the registers' old contents.
-__device__ __forceinline__ uint32_t RemainderPair(uint32_t hpair, float x0, float x1) {
-  uint32_t d;
-  asm("v_fma_mixlo_f16 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]\n\t"
-      "v_fma_mixhi_f16 %0, %1, -1.0, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
-      : "=&v"(d)
-      : "v"(hpair), "v"(x0), "v"(x1));
-  return d;
-}
+// conversions.) The compiler does not count instructions inside the block as
+// vector ALU writes, so the wait states that it would put between a
+// transcendental result and its use, and between the last write and a matrix
+// instruction that reads it, are the block's own: without the closing one a
+// schedule that multiplies at once reads the registers' old contents.
 __device__ __forceinline__ void SplitPair(const float (&x)[8], F16x8* h, F16x8* l) {
 #pragma unroll
   for (int j = 0; j < 8; ++j) (*h)[j] = static_cast<_Float16>(x[j]);
   typedef unsigned int U32x4v __attribute__((ext_vector_type(4)));
   const U32x4v hw = __builtin_bit_cast(U32x4v, *h);
-  U32x4v lw;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) lw[k] = RemainderPair(hw[k], x[2 * k], x[2 * k + 1]);
-  asm("s_nop 1" : "+v"(lw));
+  uint32_t l0, l1, l2, l3;
+  asm("s_nop 0\n\t"
+      "v_fma_mixlo_f16 %0, %4, -1.0, %8 op_sel_hi:[1,0,0]\n\t"
+      "v_fma_mixhi_f16 %0, %4, -1.0, %9 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
+      "v_fma_mixlo_f16 %1, %5, -1.0, %10 op_sel_hi:[1,0,0]\n\t"
+      "v_fma_mixhi_f16 %1, %5, -1.0, %11 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
+      "v_fma_mixlo_f16 %2, %6, -1.0, %12 op_sel_hi:[1,0,0]\n\t"
+      "v_fma_mixhi_f16 %2, %6, -1.0, %13 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
+      "v_fma_mixlo_f16 %3, %7, -1.0, %14 op_sel_hi:[1,0,0]\n\t"
+      "v_fma_mixhi_f16 %3, %7, -1.0, %15 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
+      "s_nop 1"
+      : "=&v"(l0), "=&v"(l1), "=&v"(l2), "=&v"(l3)
+      : "v"(hw[0]), "v"(hw[1]), "v"(hw[2]), "v"(hw[3]), "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]),
+        "v"(x[5]), "v"(x[6]), "v"(x[7]));
+  const U32x4v lw = {l0, l1, l2, l3};
   *l = __builtin_bit_cast(F16x8, lw);
 }
 
@@ -910,6 +921,187 @@ __device__ __forceinline__ F16x8 SplitTerm(float (&x)[8]) {
     x[j] -= static_cast<float>(h[j]);
   }
   return h;
+}
+
+// A query row as the matrix core's operand (B of the scores): lane (col, hf) holds
+// its own query's dims, the two terms of q 2^e scale log2(e); *sinv = 2^-e.
+__device__ __forceinline__ void FaLoadQ(const float* __restrict__ qrow, bool qvalid, float scale, int hf,
+                                        F16x8 (&qb)[2][8], float* sinv) {
+  // ---- q row: this lane holds dims 16 s + 8 hf + j (s = 0..7), the partner lane the rest
+  float qv[8][8];
+  float amax = 0.0f;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
+    if (qvalid) {
+      a = *reinterpret_cast<const float4*>(qrow + 16 * s + 8 * hf);
+      b = *reinterpret_cast<const float4*>(qrow + 16 * s + 8 * hf + 4);
+    }
+    qv[s][0] = a.x; qv[s][1] = a.y; qv[s][2] = a.z; qv[s][3] = a.w;
+    qv[s][4] = b.x; qv[s][5] = b.y; qv[s][6] = b.z; qv[s][7] = b.w;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(qv[s][j]));
+  }
+  amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+  int e = 0;
+  if (amax > 0.0f && amax <= 3.0e38f) e = 6 - ilogbf(amax);  // max |q| * 2^e in [64, 128)
+  if (e > 120) e = 120;  // 2^e stays finite (a row below 2^-114 scores 0 either way)
+  // Scores are kept in log2 units, so each exponential is one v_exp_f32:
+  // p = 2^(s2 - m2) = e^(s - m). The score scale (1 / sqrt(d) times log2(e))
+  // is applied to q before the split (one fp32 rounding, ~2^-24, under the
+  // split's ~2^-23): q 2^e scale log2(e) lies in [8, 17), well inside fp16's
+  // range for both terms. The matrix cores return s2 2^e, and the exponent
+  // s2 - m2 is formed as fma(s2 2^e, 2^-e, -m2), exact scaling and one rounding.
+  const float qmul = ldexpf(scale * 1.44269504088896340736f, e);
+  *sinv = ldexpf(1.0f, -e);
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      qv[s][j] *= qmul;
+      // the rounded product, and not the exact one: given the choice the compiler
+      // rounds q qmul to fp16 in one step for one use and in two for another, and
+      // where they differ the remainder belongs to another first term (a row in
+      // 300 was off by 1e-4 relative)
+      asm("" : "+v"(qv[s][j]));
+    }
+    qb[0][s] = SplitTerm(qv[s]);
+    qb[1][s] = SplitTerm(qv[s]);
+  }
+}
+
+// One block of 32 kTiles keys for a wave's 32 queries, in two steps. First the scores
+// S^T = K . Q^T; k(mt, s) is the operand of key tile mt, dims 16 s .. + 15. The
+// smallest term comes first; kFine: in two halves of the dims, all of a half's small
+// terms before its large ones, so that few sums round at full size (for a second read
+// of the keys).
+template <int kTiles, bool kFine, class KOperand>
+__device__ __forceinline__ void FaScores(const KOperand& k, const F16x8 (&qb)[2][8], F32x16 (&st)[kTiles]) {
+#pragma unroll
+  for (int mt = 0; mt < kTiles; ++mt) st[mt] = F32x16{};
+  if constexpr (kFine) {
+    F32x16 sh[kTiles];
+#pragma unroll
+    for (int mt = 0; mt < kTiles; ++mt) sh[mt] = F32x16{};
+#pragma unroll
+    for (int t = 1; t >= 0; --t)
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int mt = 0; mt < kTiles; ++mt) {
+          st[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(k(mt, s), qb[t][s], st[mt], 0, 0, 0);
+          sh[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(k(mt, s + 4), qb[t][s + 4], sh[mt], 0, 0, 0);
+        }
+#pragma unroll
+    for (int mt = 0; mt < kTiles; ++mt) st[mt] += sh[mt];
+    return;
+  }
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+#pragma unroll
+    for (int mt = 0; mt < kTiles; ++mt) {
+      const F16x8 a = k(mt, s);
+      st[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qb[1][s], st[mt], 0, 0, 0);
+      st[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qb[0][s], st[mt], 0, 0, 0);
+    }
+  }
+}
+
+// Then the online softmax and P.V into (o, m, l); v(ks, dt) is the operand of dims
+// 32 dt .. + 31 and the lane's keys of step ks (16 ks + 4 hf + 0..3 and + 8..11).
+// masked: some query of the wave does not see the whole block, or is none; then keys
+// at offsets up to rel64 count. kFine: the block's own sum first, all of its small
+// terms before its large ones, and one addition at o's size.
+template <int kTiles, bool kFine, class VOperand>
+__device__ __forceinline__ void FaAttend(const VOperand& v, F32x16 (&st)[kTiles], float sinv, bool masked, int64_t rel64,
+                                         int hf, F32x16 (&o)[4], float& m, float& l) {
+  // ---- online softmax: register r of tile mt is key 32 mt + (r % 4) + 8 (r / 4) + 4 hf
+  // of the block; the causal test is on that offset (32-bit)
+  // (a block wholly below every query of the wave, all of them valid, needs no mask)
+  float bmax = -INFINITY;
+  if (!masked) {
+#pragma unroll
+    for (int mt = 0; mt < kTiles; ++mt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) bmax = fmaxf(bmax, st[mt][r]);
+  } else {
+    const int32_t rel = static_cast<int32_t>(rel64 < 32 * kTiles ? rel64 : 32 * kTiles);  // offsets <= rel are visible
+#pragma unroll
+    for (int mt = 0; mt < kTiles; ++mt) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int32_t off = 32 * mt + (r & 3) + 8 * (r >> 2) + 4 * hf;
+        const float sc = off <= rel ? st[mt][r] : -INFINITY;
+        st[mt][r] = sc;
+        bmax = fmaxf(bmax, sc);
+      }
+    }
+  }
+  bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64)) * sinv;  // exact: a power of two
+  // The running max m moves only when a block's max exceeds it by more than
+  // kFaLazyLog2, so p <= 2^kFaLazyLog2 and most blocks rescale nothing (o and
+  // l are relative to whatever m is; the final o / l does not depend on it).
+  const float mn = bmax > m + kFaLazyLog2 ? bmax : m;
+  // 2^(-inf) = 0: masked scores give p = 0 once the row has a finite max;
+  // before that (mn = -inf) the block contributes nothing
+  const float base = mn == -INFINITY ? 0.0f : mn;
+  if (__builtin_amdgcn_ballot_w64(mn != m) != 0) {  // some row of the wave moved
+    const float corr = __builtin_amdgcn_exp2f(m - base);  // 1 where m stays; 0 on a row's first live block
+    l *= corr;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) o[dt] *= corr;
+  }
+  float psum = 0.0f;
+#pragma unroll
+  for (int mt = 0; mt < kTiles; ++mt) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(st[mt][r], sinv, -base));
+      st[mt][r] = p;
+      psum += p;
+    }
+  }
+  psum += __shfl_xor(psum, 32, 64);
+  l += psum;
+  m = mn;
+
+  // ---- O^T += V^T . P^T: key step ks takes registers 8 (ks % 2) .. + 7 of tile ks / 2
+  const auto split = [&](int ks, F16x8* ph, F16x8* pl) {
+    float pr[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) pr[j] = st[ks >> 1][8 * (ks & 1) + j];
+    SplitPair(pr, ph, pl);
+  };
+  if constexpr (kFine) {
+    F16x8 p[2][2 * kTiles];
+#pragma unroll
+    for (int ks = 0; ks < 2 * kTiles; ++ks) split(ks, &p[0][ks], &p[1][ks]);
+#pragma unroll
+    for (int d2 = 0; d2 < 4; d2 += 2) {
+      F32x16 sum[2] = {F32x16{}, F32x16{}};
+#pragma unroll
+      for (int t = 1; t >= 0; --t)
+#pragma unroll
+        for (int ks = 0; ks < 2 * kTiles; ++ks)
+#pragma unroll
+          for (int d = 0; d < 2; ++d)
+            sum[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v(ks, d2 + d), p[t][ks], sum[d], 0, 0, 0);
+      o[d2] += sum[0];
+      o[d2 + 1] += sum[1];
+    }
+    return;
+  }
+#pragma unroll
+  for (int ks = 0; ks < 2 * kTiles; ++ks) {
+    F16x8 ph, pl;
+    split(ks, &ph, &pl);
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) {
+      const F16x8 a = v(ks, dt);
+      o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pl, o[dt], 0, 0, 0);
+      o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, ph, o[dt], 0, 0, 0);
+    }
+  }
 }
 
 // Dispatch order of the prefill workgroups. Workgroup g takes query head g %
@@ -930,13 +1122,15 @@ struct FaOrder {
 // others get an unnormalised partial (o, m, l) per live chunk in `part`, laid
 // out as the decode partials ([token][head][chunk]), which AttnMergeRowsKernel
 // combines.
+template <bool kDirect>
 __global__ __launch_bounds__(256, 2) void AttnPrefillMfmaKernel(
     const float* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc, int64_t max_seq,
     int32_t n_heads, int32_t group, float scale, int64_t pos0_val, const int64_t* __restrict__ pos0_dev, int64_t seq,
     int32_t n_chunks, int64_t chunk_len, int32_t tiles, float* __restrict__ out, float* __restrict__ part,
     FaOrder order, uint32_t* __restrict__ cnt) {
-  __shared__ __attribute__((aligned(16))) _Float16 ks[kFaKeys * kFaKStride];
-  __shared__ __attribute__((aligned(16))) _Float16 vs[kFaKeys * kFaVStride];
+  // an array each: a read waits only for the loads into its own array
+  __shared__ __attribute__((aligned(16))) _Float16 ks0[kFaKeys * kD], ks1[kFaKeys * kD];
+  __shared__ __attribute__((aligned(16))) _Float16 vs0[kFaKeys * kD], vs1[kFaKeys * kD];
   const int lane = threadIdx.x & 63;
   const int wv = threadIdx.x >> 6;
   const int hf = lane >> 5;    // which half of the keys / dims this lane holds
@@ -966,48 +1160,9 @@ __global__ __launch_bounds__(256, 2) void AttnPrefillMfmaKernel(
   const bool qvalid = tq < seq;
   const int64_t qpos = pos0 + tq;
 
-  // ---- q row: this lane holds dims 16 s + 8 hf + j (s = 0..7), the partner lane the rest
-  float qv[8][8];
-  const float* qrow = q + (tq * n_heads + h) * kD;
-  float amax = 0.0f;
-#pragma unroll
-  for (int s = 0; s < 8; ++s) {
-    float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
-    if (qvalid) {
-      a = *reinterpret_cast<const float4*>(qrow + 16 * s + 8 * hf);
-      b = *reinterpret_cast<const float4*>(qrow + 16 * s + 8 * hf + 4);
-    }
-    qv[s][0] = a.x; qv[s][1] = a.y; qv[s][2] = a.z; qv[s][3] = a.w;
-    qv[s][4] = b.x; qv[s][5] = b.y; qv[s][6] = b.z; qv[s][7] = b.w;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(qv[s][j]));
-  }
-  amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
-  int e = 0;
-  if (amax > 0.0f && amax <= 3.0e38f) e = 6 - ilogbf(amax);  // max |q| * 2^e in [64, 128)
-  // Scores are kept in log2 units, so each exponential is one v_exp_f32:
-  // p = 2^(s2 - m2) = e^(s - m). The score scale (1 / sqrt(d) times log2(e))
-  // is applied to q before the split (one fp32 rounding, ~2^-24, under the
-  // split's ~2^-23): q 2^e scale log2(e) lies in [8, 17), well inside fp16's
-  // range for both terms. The matrix cores return s2 2^e, and the exponent
-  // s2 - m2 is formed as fma(s2 2^e, 2^-e, -m2), exact scaling and one rounding.
-  const float qmul = ldexpf(scale * 1.44269504088896340736f, e);
-  const float sinv = ldexpf(1.0f, -e);
   F16x8 qb[2][8];
-#pragma unroll
-  for (int s = 0; s < 8; ++s) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      qv[s][j] *= qmul;
-      // the rounded product, and not the exact one: given the choice the compiler
-      // rounds q qmul to fp16 in one step for one use and in two for another, and
-      // where they differ the remainder belongs to another first term (one row in
-      // 300 was off by 1e-4 relative)
-      asm("" : "+v"(qv[s][j]));
-    }
-    qb[0][s] = SplitTerm(qv[s]);
-    qb[1][s] = SplitTerm(qv[s]);
-  }
+  float sinv;
+  FaLoadQ(q + (tq * n_heads + h) * kD, qvalid, scale, hf, qb, &sinv);
 
   F32x16 o[4];
 #pragma unroll
@@ -1025,120 +1180,55 @@ __global__ __launch_bounds__(256, 2) void AttnPrefillMfmaKernel(
   if (klo > last_key) return;  // no key of this chunk is visible to the tile (uniform: before any barrier)
   const int64_t kend = klo + chunk_len;
 
-  for (int64_t kb = klo; kb <= last_key && kb < kend; kb += kFaKeys) {
-    __syncthreads();  // the previous block is consumed
-    {
-      // thread t: key t / 4, dims 32 (t % 4) .. + 31 of K and V
-      const int key = threadIdx.x >> 2;
-      const int part = threadIdx.x & 3;
-      // rows past the causal limit repeat the last visible row: their scores are
-      // masked, so p = 0 meets finite values
-      const int64_t j = kb + key < last_key ? kb + key : last_key;
-      uint4 kw[4], vw[4];
-      const uint4* kr = reinterpret_cast<const uint4*>(kbase + j * kD + 32 * part);
-      const uint4* vr = reinterpret_cast<const uint4*>(vbase + j * kD + 32 * part);
+  // Load j of a wave takes rows 16 j + 4 wv + lane / 16 of the block, to LDS piece lane
+  // % 16 of 16 bytes: piece p of row r lies at p ^ r % 16 (K), p ^ 4 (r % 4) (V), which
+  // spreads both operands' reads over the banks. Rows past the causal limit repeat the
+  // last visible row: their scores are masked, so p = 0 meets finite values.
+  const int lrow = lane >> 4;
+  const int kpiece = 8 * ((lane & 15) ^ (4 * wv + lrow));
+  const int vpiece = 8 * ((lane & 15) ^ (4 * lrow));
+  const auto stage = [&](int64_t kb, _Float16* kto, _Float16* vto) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        kw[i] = kr[i];
-        vw[i] = vr[i];
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(&ks[key * kFaKStride + 32 * part + 8 * i]) = kw[i];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(&vs[key * kFaVStride + 32 * part + 8 * i]) = vw[i];
-    }
-    __syncthreads();
-    if (kb > wave_last) continue;  // every query of this wave is before the block (uniform per wave)
-
-    // ---- S^T = K . Q^T (the smallest term first)
-    F32x16 st[2] = {F32x16{}, F32x16{}};
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-#pragma unroll
-      for (int mt = 0; mt < 2; ++mt) {
-        const F16x8 a = *reinterpret_cast<const F16x8*>(&ks[(32 * mt + col) * kFaKStride + 16 * s + 8 * hf]);
-        st[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qb[1][s], st[mt], 0, 0, 0);
-        st[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qb[0][s], st[mt], 0, 0, 0);
+    for (int j = 0; j < kFaKeys / 16; ++j) {
+      const int row = 16 * j + 4 * wv;
+      const int64_t key = kb + row + lrow < last_key ? kb + row + lrow : last_key;
+      if constexpr (kDirect) {
+        LoadToLds(kbase + key * kD + kpiece, kto + row * kD);
+        LoadToLds(vbase + key * kD + vpiece, vto + row * kD);
+      } else {
+        *reinterpret_cast<uint4*>(kto + row * kD + 8 * lane) = *reinterpret_cast<const uint4*>(kbase + key * kD + kpiece);
+        *reinterpret_cast<uint4*>(vto + row * kD + 8 * lane) = *reinterpret_cast<const uint4*>(vbase + key * kD + vpiece);
       }
     }
-
-    // ---- online softmax: register r of tile mt is key kb + 32 mt + (r % 4) + 8 (r / 4) + 4 hf;
-    // the causal test on the key's offset in the block (32-bit)
-    // (a block wholly below every query of the wave, all of them valid, needs no mask)
-    float bmax = -INFINITY;
-    if (kb + kFaKeys - 1 <= wave_first && wave_full) {
-#pragma unroll
-      for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) bmax = fmaxf(bmax, st[mt][r]);
-    } else {
-      const int64_t rel64 = qvalid ? qpos - kb : -1;
-      const int32_t rel = static_cast<int32_t>(rel64 < 64 ? rel64 : 64);  // offsets <= rel are visible
-#pragma unroll
-      for (int mt = 0; mt < 2; ++mt) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int32_t off = 32 * mt + (r & 3) + 8 * (r >> 2) + 4 * hf;
-          const float sc = off <= rel ? st[mt][r] : -INFINITY;
-          st[mt][r] = sc;
-          bmax = fmaxf(bmax, sc);
-        }
-      }
-    }
-    bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64)) * sinv;  // exact: a power of two
-    // The running max m moves only when a block's max exceeds it by more than
-    // kFaLazyLog2, so p <= 2^kFaLazyLog2 and most blocks rescale nothing (o and
-    // l are relative to whatever m is; the final o / l does not depend on it).
-    const float mn = bmax > m + kFaLazyLog2 ? bmax : m;
-    // 2^(-inf) = 0: masked scores give p = 0 once the row has a finite max;
-    // before that (mn = -inf) the block contributes nothing
-    const float base = mn == -INFINITY ? 0.0f : mn;
-    if (__builtin_amdgcn_ballot_w64(mn != m) != 0) {  // some row of the wave moved
-      const float corr = __builtin_amdgcn_exp2f(m - base);  // 1 where m stays; 0 on a row's first live block
-      l *= corr;
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt) o[dt] *= corr;
-    }
-    float psum = 0.0f;
-#pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(st[mt][r], sinv, -base));
-        st[mt][r] = p;
-        psum += p;
-      }
-    }
-    psum += __shfl_xor(psum, 32, 64);
-    l += psum;
-    m = mn;
-
-    // ---- O^T += V^T . P^T: key step ks takes registers 8 (ks % 2) .. + 7 of tile ks / 2
-#pragma unroll
-    for (int ks2 = 0; ks2 < 4; ++ks2) {
-      const int mt = ks2 >> 1;
-      const int rb = 8 * (ks2 & 1);
-      float pr[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) pr[j] = st[mt][rb + j];
-      F16x8 ph, pl;
-      SplitPair(pr, &ph, &pl);
-      const int koff = 32 * mt + 16 * (ks2 & 1) + 4 * hf;  // keys koff + 0..3 and koff + 8..11
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt) {
-        // V^T fragment of dim 32 dt + col from V rows by transposing reads: in
-        // each 16-lane group, lane j points at key koff + j / 4 (resp. + 8),
-        // dims 32 dt + 16 (col / 16) + 4 (j % 4) .. + 3, and receives dim
-        // 32 dt + col of keys koff .. koff + 3 (resp. koff + 8 .. + 11)
-        const int gj = lane & 15;
-        const int vd = 32 * dt + (col & 16) + 4 * (gj & 3);
-        const F16x4 lo = VTr(&vs[(koff + (gj >> 2)) * kFaVStride + vd]);
-        const F16x4 hi = VTr(&vs[(koff + 8 + (gj >> 2)) * kFaVStride + vd]);
-        const F16x8 a = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pl, o[dt], 0, 0, 0);
-        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, ph, o[dt], 0, 0, 0);
-      }
-    }
+  };
+  const int k_lane = col * kD + 8 * (hf ^ (col & 15));
+  // V^T fragment of dim 32 dt + col from V rows by transposing reads: in each 16-lane
+  // group, lane j points at key koff + j / 4 (resp. + 8), dims 32 dt + 16 (col / 16) +
+  // 4 (j % 4) .. + 3, and receives dim 32 dt + col of keys koff .. koff + 3 (resp.
+  // koff + 8 .. + 11)
+  const int gj = lane & 15;
+  const int v_lane = (4 * hf + (gj >> 2)) * kD + 8 * ((2 * (col >> 4) + ((gj & 3) >> 1)) ^ (4 * (gj >> 2))) + 4 * (gj & 1);
+  // The block at kb from one pair of arrays, the next one on its way to the other.
+  const auto block = [&](int64_t kb, const _Float16* ks, const _Float16* vs, _Float16* knext, _Float16* vnext) {
+    if constexpr (kDirect) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();  // the block is there, and nobody reads the other arrays any more
+    if (kb + kFaKeys <= last_key && kb + kFaKeys < kend) stage(kb + kFaKeys, knext, vnext);
+    if (kb > wave_last) return;  // every query of this wave is before the block (uniform per wave)
+    F32x16 st[2];
+    FaScores<2, false>(
+        [&](int mt, int s) { return *reinterpret_cast<const F16x8*>(&ks[(k_lane ^ (16 * s)) + 32 * mt * kD]); }, qb, st);
+    const auto v_operand = [&](int ks2, int dt) {
+      const _Float16* const at = &vs[(v_lane ^ (32 * dt)) + 16 * ks2 * kD];
+      const F16x4 lo = VTr(at);
+      const F16x4 hi = VTr(at + 8 * kD);
+      return F16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    };
+    FaAttend<2, false>(v_operand, st, sinv, kb + kFaKeys - 1 > wave_first || !wave_full, qvalid ? qpos - kb : -1, hf, o, m, l);
+  };
+  stage(klo, ks0, vs0);
+  for (int64_t kb = klo; kb <= last_key && kb < kend; kb += 2 * kFaKeys) {
+    block(kb, ks0, vs0, ks1, vs1);
+    if (kb + kFaKeys <= last_key && kb + kFaKeys < kend) block(kb + kFaKeys, ks1, vs1, ks0, vs0);
   }
 
   // ---- out[tq][h][dim]: register r of tile dt is dim 32 dt + (r % 4) + 8 (r / 4) + 4 hf
@@ -1293,6 +1383,179 @@ __global__ __launch_bounds__(256, 2) void AttnPrefillMfmaKernel(
   }
   // every workgroup of the (tile, head) has counted in: ready for the next call
   if (threadIdx.x == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// ---------------------------------------------------------------- a few tokens over a long cache
+//
+// Short turns (2 to kFaMinTokens - 1 tokens): the workgroup of (32-token tile, query
+// head) takes all of the tile's keys, each of its waves every kTurnWaves-th block of
+// kTurnKeys, and the waves' partials meet in LDS: no partials in memory, whatever the
+// stream. K and V go straight to LDS of the wave's own (no barrier in the loop), the
+// next block's keys while the values are used and the next values during the scores;
+// rows are 256 bytes, their 16-byte pieces exchanged by the row's number (the lanes'
+// sources are chosen so), which spreads both operands' reads over the banks. What
+// bounds it is the serial chain of a wave's blocks. 45 tokens at position 1500 (16 / 8
+// heads): 39 us with a wave per (token, kv head, key chunk), which reads the cache 45
+// times, 24 here.
+constexpr int kTurnRows = 32;
+constexpr int kTurnKeys = 32;
+constexpr int kTurnWaves = 8;
+
+__global__ __launch_bounds__(64 * kTurnWaves, 1) void AttnTurnKernel(
+    const float* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc, int64_t max_seq,
+    int32_t n_heads, int32_t group, float scale, int64_t pos0_val, const int64_t* __restrict__ pos0_dev, int64_t seq,
+    float* __restrict__ out) {
+  __shared__ __attribute__((aligned(16))) _Float16 lds_k[kTurnWaves * kTurnKeys * kD], lds_v[kTurnWaves * kTurnKeys * kD];
+  __shared__ float wm[kTurnWaves][kTurnRows], wl[kTurnWaves][kTurnRows];
+  static_assert(sizeof(float) * kTurnWaves / 2 * kTurnRows * kD <= sizeof(lds_k), "the waves' outputs fit where K and V were");
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int hf = lane >> 5;
+  const int col = lane & 31;
+  // heads sharing a kv head n_kv apart: with 8 of them each stays on one XCD and its L2
+  const int n_kv = n_heads / group;
+  const int tile = static_cast<int>(blockIdx.x) / n_heads;
+  const int slot = static_cast<int>(blockIdx.x) - tile * n_heads;
+  const int kh = slot % n_kv;
+  const int h = kh * group + slot / n_kv;
+  const int64_t t_first = kTurnRows * tile;
+  const int64_t tq = t_first + col;
+  const bool qvalid = tq < seq;
+  const int64_t pos0 = ReadPos0(pos0_val, pos0_dev);
+  const bool full = t_first + kTurnRows <= seq;
+  const int64_t last_key = pos0 + (full ? t_first + kTurnRows : seq) - 1;  // the tile's causal limit
+
+  // a block's rows: load j takes rows 4 j + lane / 16, to piece lane % 16 (rows past
+  // the causal limit repeat the last visible one: p = 0 meets finite values)
+  _Float16* const ks = lds_k + wv * (kTurnKeys * kD);
+  _Float16* const vs = lds_v + wv * (kTurnKeys * kD);
+  const uint16_t* const kbase = kc + kh * max_seq * kD;
+  const uint16_t* const vbase = vc + kh * max_seq * kD;
+  const uint32_t lrow = static_cast<uint32_t>(lane) >> 4;
+  const auto load = [&](const uint16_t* base, int64_t kb, uint32_t piece, uint32_t turn, _Float16* to) {
+    const uint32_t visible = static_cast<uint32_t>(last_key - kb < kTurnKeys ? last_key - kb : kTurnKeys);
+#pragma unroll
+    for (uint32_t j = 0; j < kTurnKeys / 4; ++j) {
+      const uint32_t row = 4 * j + lrow < visible ? 4 * j + lrow : visible;
+      LoadToLds(base + kb * kD + (row * kD + 8 * (piece ^ (turn * j & 15))), to + 4 * j * kD);
+    }
+  };
+  const auto load_k = [&](int64_t kb) { load(kbase, kb, (lane & 15) ^ lrow, 4, ks); };      // piece ^ row % 16
+  const auto load_v = [&](int64_t kb) { load(vbase, kb, (lane & 15) ^ (4 * lrow), 0, vs); };  // piece ^ 4 (row % 4)
+  // in the loop the addresses are formed anew from these (kept, all of them would spill)
+  int k_lane = col * kD + 8 * (hf ^ (col & 15));
+  const int gj = lane & 15;  // V^T by transposing reads, as in AttnPrefillMfmaKernel
+  int v_lane = (4 * hf + (gj >> 2)) * kD + 8 * ((2 * (col >> 4) + ((gj & 3) >> 1)) ^ (4 * (gj >> 2))) + 4 * (gj & 1);
+  const auto k_operand = [&](int, int s) { return *reinterpret_cast<const F16x8*>(&ks[k_lane ^ (16 * s)]); };
+  const auto v_operand = [&](int step, int dt) {
+    const _Float16* const at = &vs[(v_lane ^ (32 * dt)) + 16 * step * kD];
+    const F16x4 lo = VTr(at);
+    const F16x4 hi = VTr(at + 8 * kD);
+    return F16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+  };
+
+  F16x8 qb[2][8];
+  float sinv;
+  FaLoadQ(q + ((qvalid ? tq : 0) * n_heads + h) * kD, qvalid, scale, hf, qb, &sinv);
+  F32x16 o[4];
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt) o[dt] = F32x16{};
+  float m = -INFINITY, l = 0.0f;
+  int64_t kb = kTurnKeys * wv;
+  if (kb <= last_key) {
+    load_k(kb);
+    load_v(kb);
+  }
+  for (; kb <= last_key; kb += kTurnKeys * kTurnWaves) {
+    const bool more = kb + kTurnKeys * kTurnWaves <= last_key;
+    asm("" : "+v"(k_lane), "+v"(v_lane));
+    static_assert(kTurnKeys / 4 == 8, "the waits below count a block's loads");
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // the keys are there, the values may be under way
+    F32x16 st[1];
+    FaScores<1, true>(k_operand, qb, st);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the keys are read before the next ones are written
+    if (more) {
+      load_k(kb + kTurnKeys * kTurnWaves);
+      asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    const bool partly = kb + kTurnKeys - 1 > pos0 + t_first;  // some token does not see the whole block
+    const int64_t seen = qvalid ? pos0 + tq - kb : -1;        // offsets the lane's token sees, at most
+    // 0 times a value that is not finite would reach the tokens before it: such
+    // values count as 0 in the products and are added for the tokens that see them
+    uint64_t broken = 0;
+    if (partly) {
+#pragma unroll 1
+      for (int j = 0; j < kTurnKeys / 4; ++j) {
+        F16x8* const at = reinterpret_cast<F16x8*>(&vs[4 * j * kD + 8 * lane]);
+        F16x8 v = *at;
+        bool hit = false;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const bool bad = !(fabsf(static_cast<float>(v[i])) <= 65504.0f);
+          v[i] = bad ? static_cast<_Float16>(0.0f) : v[i];
+          hit |= bad;
+        }
+        if (hit) *at = v;
+        broken |= __builtin_amdgcn_ballot_w64(hit);
+      }
+    }
+    FaAttend<1, true>(v_operand, st, sinv, partly || !full, seen, hf, o, m, l);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (broken != 0) {
+#pragma unroll 1
+      for (int64_t key = 0; key < kTurnKeys && key <= seen; ++key) {
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int dim = 32 * dt + (r & 3) + 8 * (r >> 2) + 4 * hf;
+            const float v = static_cast<float>(__builtin_bit_cast(_Float16, vbase[(kb + key) * kD + dim]));
+            o[dt][r] += fabsf(v) <= 65504.0f ? 0.0f : v;
+          }
+      }
+    }
+    if (more) load_v(kb + kTurnKeys * kTurnWaves);
+  }
+
+  // ---- the waves' partials: weights against the common maximum, outputs summed in wave order
+  if (hf == 0) {
+    wm[wv][col] = m;
+    wl[wv][col] = l;
+  }
+  __syncthreads();
+  float mx = -INFINITY, L = 0.0f;
+#pragma unroll
+  for (int w = 0; w < kTurnWaves; ++w) mx = fmaxf(mx, wm[w][col]);
+#pragma unroll
+  for (int w = 0; w < kTurnWaves; ++w) {
+    L = __builtin_fmaf(wl[w][col], wm[w][col] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(wm[w][col] - mx), L);
+  }
+  const float f = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mx);
+  // [wave][float4 8 dt + 2 g + hf][row], half of the waves where the keys were and half where the values were
+  const auto sums = [&](int w) { return reinterpret_cast<float4*>(w < kTurnWaves / 2 ? lds_k : lds_v) + w % (kTurnWaves / 2) * 32 * kTurnRows; };
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      sums(wv)[(8 * dt + 2 * g + hf) * kTurnRows + col] =
+          make_float4(o[dt][4 * g] * f, o[dt][4 * g + 1] * f, o[dt][4 * g + 2] * f, o[dt][4 * g + 3] * f);
+  __syncthreads();
+  if (!qvalid) return;
+  // wave wv finishes dims 16 wv .. + 15: 4 of them, 8 g + 4 hf .. + 3, in each lane
+  const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+  float* orow = out + (tq * n_heads + h) * kD + 16 * wv + 4 * hf;
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    float4 acc = sums(0)[(4 * wv + 2 * g + hf) * kTurnRows + col];
+#pragma unroll
+    for (int w = 1; w < kTurnWaves; ++w) {
+      const float4 v = sums(w)[(4 * wv + 2 * g + hf) * kTurnRows + col];
+      acc = make_float4(acc.x + v.x, acc.y + v.y, acc.z + v.z, acc.w + v.w);
+    }
+    *reinterpret_cast<float4*>(orow + 8 * g) = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+  }
 }
 
 // ---------------------------------------------------------------- partials buffer
@@ -1551,6 +1814,49 @@ void LaunchDecodeGroup(const ModelMeta& c, const Pos0Arg& p0, const float* q_dev
   }
 }
 
+// What the decode kernel takes for several tokens, in us: it reads the cache once per
+// (token, kv head), so n_kv tokens positions times a rate that grows with the heads of a
+// group, and more once the (token, kv head) pairs leave fewer key chunks each (measured:
+// 16 / 8 heads, 21 tokens at 1500 17 us, 31 at 3000 46, 45 at 1500 39; 32 / 8 heads, 21
+// at 3000 42, 45 at 1500 63).
+double DecodeUs(const ModelMeta& c, int64_t seq, int64_t positions) {
+  const int group = c.n_heads / c.n_kv_heads;
+  const double units = static_cast<double>(seq * c.n_kv_heads);
+  const double rate = (group <= 1 ? 3.5e-5 : group <= 2 ? 4.4e-5 : 7.2e-5) * (units >= 256 ? 1.35 : 1.0);
+  return 5.0 + units * static_cast<double>(positions) * rate;
+}
+
+// Calls for AttnTurnKernel: 2 to kFaMinTokens - 1 tokens where the decode kernel takes
+// longer than its 7 us and 2.35 us a block of every wave (with a tenth to spare, for
+// the groups measured; from 1024 positions on, where its error is no larger than the
+// decode kernel's: 2.0e-7 and 2.3e-7 for 45 tokens at 1500), with the alignment of the
+// 16-byte loads and stores. A call whose split decode the fixed region is too small
+// for stays with it, and is refused.
+bool TurnWins(const ModelMeta& c, const float* q_dev, int64_t seq, const uint16_t* v_layer, const float* out_dev,
+              int64_t positions, const PartialsSink& sink) {
+  const int group = c.n_heads / c.n_kv_heads;
+  const int64_t groups = (seq + kTurnRows - 1) / kTurnRows * c.n_heads;
+  if (seq < 2 || seq >= kFaMinTokens || positions < 1024 || (group != 1 && group != 2 && group != 4) || groups > 256 ||
+      ((reinterpret_cast<uintptr_t>(q_dev) | reinterpret_cast<uintptr_t>(v_layer) |
+        reinterpret_cast<uintptr_t>(out_dev)) & 15u) != 0) {
+    return false;
+  }
+  int32_t n_chunks;
+  int64_t chunk_len;
+  PlanGroupChunks(seq * c.n_kv_heads, positions, &n_chunks, &chunk_len);
+  const int64_t n_groups = (n_chunks + kFusedWaves - 1) / kFusedWaves;
+  if (n_groups > 1 && static_cast<size_t>(seq * c.n_heads * n_groups * kPartFloats) > sink.Capacity()) return false;
+  const int64_t blocks = (positions + kTurnKeys * kTurnWaves - 1) / (kTurnKeys * kTurnWaves);
+  return 1.1 * (7.0 + 2.35 * static_cast<double>(blocks)) < DecodeUs(c, seq, positions);
+}
+
+void LaunchTurn(const ModelMeta& c, const Pos0Arg& p0, const float* q_dev, int64_t seq, const uint16_t* k_layer,
+                const uint16_t* v_layer, int64_t max_seq, float scale, float* out_dev) {
+  Launch("AttnTurnKernel", AttnTurnKernel, dim3(static_cast<unsigned>((seq + kTurnRows - 1) / kTurnRows * c.n_heads)),
+         dim3(64 * kTurnWaves), q_dev, k_layer, v_layer, max_seq, c.n_heads, c.n_heads / c.n_kv_heads, scale, p0.value,
+         p0.dev, seq, out_dev);
+}
+
 // GpuAttentionFromCache with the chunk partials taken from `sink`.
 void AttentionFromCache(const ModelMeta& c, int64_t pos0, const float* q_dev, int64_t seq, const uint16_t* k_layer,
                         const uint16_t* v_layer, int64_t max_seq, float* out_dev, int64_t sh_positions,
@@ -1574,6 +1880,10 @@ void AttentionFromCache(const ModelMeta& c, int64_t pos0, const float* q_dev, in
   int64_t chunk_len;
   PlanChunks(pairs, positions, &n_chunks, &chunk_len);
   const Pos0Arg p0 = Pos0ForLaunch(pos0);
+  if (TurnWins(c, q_dev, seq, v_layer, out_dev, positions, sink)) {
+    LaunchTurn(c, p0, q_dev, seq, k_layer, v_layer, max_seq, scale, out_dev);
+    return;
+  }
   if (seq >= kFaMinTokens) {
     // Key chunks of at most max(8, total / 512) key blocks per workgroup (two
     // workgroups per CU), counted over the position budget; the partials stay
@@ -1632,8 +1942,11 @@ void AttentionFromCache(const ModelMeta& c, int64_t pos0, const float* q_dev, in
     uint32_t* cnt = fa_chunks > 1 && fa_chunks <= kFaFusedMaxChunks && tiles * c.n_heads <= kFaCounterSlots
                         ? sink.PrefillCounters()
                         : nullptr;
-    Launch("AttnPrefillMfmaKernel", AttnPrefillMfmaKernel, dim3(static_cast<unsigned>(n_pairs * c.n_heads)),
-           dim3(kBlockThreads), q_dev, k_layer, v_layer, max_seq, c.n_heads, c.n_heads / c.n_kv_heads, scale,
+    // straight to LDS only from 16-byte aligned rows (V's may start at any 4 bytes)
+    const bool direct = (reinterpret_cast<uintptr_t>(v_layer) & 15u) == 0;
+    Launch("AttnPrefillMfmaKernel", direct ? AttnPrefillMfmaKernel<true> : AttnPrefillMfmaKernel<false>,
+           dim3(static_cast<unsigned>(n_pairs * c.n_heads)), dim3(kBlockThreads), q_dev, k_layer, v_layer, max_seq,
+           c.n_heads, c.n_heads / c.n_kv_heads, scale,
            p0.value, p0.dev, seq, static_cast<int32_t>(fa_chunks), fa_len, static_cast<int32_t>(tiles), out_dev,
            part, order, cnt);
     if (fa_chunks > 1 && cnt == nullptr) {

@@ -1,0 +1,116 @@
+"""Short turns over a long cache (the matrix-core kernel for 2 to 63 tokens): its
+tiles' and blocks' edges against the float64 oracle, within the bound of
+tests/test_gpu_attention.py; an infinite value reaches only the tokens that see it;
+a capture laid out for a larger budget; values outside the tile's keys don't matter."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from test_gpu_attention import check, dev, host, make
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # (n_heads, n_kv_heads, max_seq, pos0, seq)
+    (16, 8, 4096, 1500, 45),
+    (16, 8, 4096, 1504, 64 - 1),   # the first token's keys end in the middle of a block
+    (32, 8, 2048, 1503, 32),       # a full tile
+    (32, 8, 2048, 2048 - 33, 33),  # one token in the second tile, full cache
+    (32, 8, 4200, 4096, 22),       # a last block of one key for some tokens
+    (8, 8, 8192, 6001, 63),        # MHA
+]
+
+
+def takes_it(gpu, call):
+    gpu.profile_start(4)
+    call()
+    gpu.profile_stop()
+    return set(gpu.profile_report()) == {"AttnTurnKernel"}
+
+
+@pytest.mark.parametrize("nh,nkv,max_seq,pos0,seq", CASES)
+def test_turn_vs_f64(gpu, ora, nh, nkv, max_seq, pos0, seq):
+    import torch
+
+    rng = np.random.default_rng(pos0 + seq + nh)
+    q, kc, vc = make(rng, nh, nkv, max_seq, seq, qscale=0.5)
+    q[seq // 2] *= 1e-42 if seq % 2 else 1e-3  # a subnormal row: every key counts alike
+    kc = kc.copy().reshape(nkv, max_seq, 128)
+    vc = vc.copy().reshape(nkv, max_seq, 128)
+    ref, smag, vmax = ora.attention_f64(q, kc.reshape(-1), vc.reshape(-1), max_seq, nh, nkv, 128, pos0, seq)
+    kc[:, pos0 + seq:] = np.float16(np.inf).view(np.uint16)
+    vc[:, pos0 + seq:] = np.float16(np.nan).view(np.uint16)
+    out = torch.full((seq + 1, nh, 128), np.nan, dtype=torch.float32, device="cuda")
+    args = (nh, nkv, 128, pos0, dev(q), seq, dev(kc.reshape(-1)), dev(vc.reshape(-1)), max_seq)
+    assert takes_it(gpu, lambda: gpu.GpuAttentionFromCache(*args, out))
+    check(host(out)[:seq], ref, smag, vmax, pos0)
+    assert torch.isnan(out[seq]).all(), "wrote past the last token"
+
+
+def test_turn_infinite_value(gpu, ora):
+    """Token 20's value row holds an infinity: tokens 0 to 19 keep their results bit for
+    bit, and from token 20 on that element is the infinity and the others are as before."""
+    import torch
+
+    nh, nkv, max_seq, pos0, seq = 16, 8, 2048, 1500, 45
+    rng = np.random.default_rng(7)
+    q, kc, vc = make(rng, nh, nkv, max_seq, seq)
+    outs = []
+    for bad in (False, True):
+        v = vc.copy().reshape(nkv, max_seq, 128)
+        v[:, pos0 + 20, 77] = np.float16(-np.inf if bad else 0.0).view(np.uint16)
+        out = torch.empty((seq, nh, 128), dtype=torch.float32, device="cuda")
+        gpu.GpuAttentionFromCache(nh, nkv, 128, pos0, dev(q), seq, dev(kc), dev(v.reshape(-1)), max_seq, out)
+        outs.append(host(out))
+    plain, got = outs
+    assert np.array_equal(plain[:20], got[:20])
+    assert np.all(got[20:, :, 77] == -np.inf)
+    assert np.array_equal(np.delete(plain, 77, axis=2), np.delete(got, 77, axis=2))
+
+
+def test_turn_captured(gpu, ora):
+    """Captured for a budget of 4096 positions and replayed at others, with eager work
+    and synchronisations in between."""
+    import torch
+
+    nh, nkv, max_seq, seq = 16, 8, 4096, 45
+    rng = np.random.default_rng(11)
+    q, kc, vc = make(rng, nh, nkv, max_seq, seq, qscale=0.5)
+    qd, kd, vd = dev(q), dev(kc), dev(vc)
+    out = torch.empty((seq, nh, 128), dtype=torch.float32, device="cuda")
+    gpu.init()
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        with gpu.ScopedEngineStream(stream):
+            graph.capture_begin()
+            gpu.GpuAttentionFromCache(nh, nkv, 128, 0, qd, seq, kd, vd, max_seq, out, max_seq)
+            graph.capture_end()
+    torch.cuda.synchronize()
+    for pos in (0, 31, 1500, 4096 - seq, 1200):
+        gpu.stage_pos0(pos)
+        torch.cuda.synchronize()
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        ref, smag, vmax = ora.attention_f64(q, kc, vc, max_seq, nh, nkv, 128, pos, seq)
+        check(host(out), ref, smag, vmax, pos)
+
+
+@pytest.mark.parametrize("seq", [64, 130])
+def test_prefill_unaligned_values(gpu, seq):
+    """The prefill kernel with the value rows at an address that is only a multiple of 4
+    bytes gives the bits of the aligned call."""
+    import torch
+
+    nh, nkv, max_seq, pos0 = 4, 2, 512, 77
+    rng = np.random.default_rng(seq)
+    q, kc, vc = make(rng, nh, nkv, max_seq, seq)
+    moved = torch.zeros(vc.size + 8, dtype=torch.int16, device="cuda")
+    moved[2:2 + vc.size] = dev(vc.reshape(-1).view(np.int16))
+    outs = [torch.empty((seq, nh, 128), device="cuda") for _ in range(2)]
+    for v, out in ((dev(vc), outs[0]), (moved[2:2 + vc.size], outs[1])):
+        gpu.GpuAttentionFromCache(nh, nkv, 128, pos0, dev(q), seq, dev(kc), v, max_seq, out)
+    assert torch.equal(*outs)
