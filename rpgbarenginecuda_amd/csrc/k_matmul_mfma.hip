@@ -580,25 +580,30 @@ __global__ __launch_bounds__(kThreads) void MatMulSplitReduceKernel(const float*
 //
 // For grids of many tiles the weights are decoded once per call instead of
 // once per token tile: DecodeWeightPlanesKernel writes fp16 operand planes
-// ([ops][rows][cols], K contiguous) and, per (row, block), (d, dmin) and
+// (in operand order, see PlanePiece) and, per (row, block), (d, dmin) and
 // m_j 2^6. Q4_K: the exact sc_j q of StageChunk. Q6_K: w = sc (q - 32) as
 // hi = w rounded to fp16 and lo = w - hi (exact; lo is nonzero only for
 // |w| > 2048, where it is +-1); the matrix cores form x_hi w_hi, x_lo w_hi and
 // x_hi w_lo and leave out x_lo w_lo, which is below 2^-22 |x w| (|x_lo| <=
 // 2^-11 |x|, |w_lo| <= 2^-11 |w|): three products instead of the four of the
 // even / odd scale split. MatMulMfmaPlanesKernel streams both operands
-// through LDS unchanged. Its workgroup is 8 waves (2 x 4) over 128
-// tokens x kPTileR rows, each wave 64 tokens x 32 kPNT rows; two LDS buffers
-// alternate every 64-column chunk, the next chunk's LDS writes and global loads
-// are issued after the first of its four K-steps, and the block-end values are
-// loaded at the block's first chunk, so one barrier per chunk is the only
-// synchronisation. For Q4_K the MFMAs, block scales and min terms of each
+// unchanged. Its workgroup is 8 waves (2 x 4) over 128 tokens x kTileR rows,
+// each wave 64 tokens x 32 kNT rows. LDS bandwidth would bound it if both operands
+// went through it (a K-step's reads and writes took as long as its products), so only
+// the activations do, straight from memory and three 64-column chunks ahead; the
+// weights lie in operand order and go from their planes to registers, a chunk ahead.
+// The block-end values are loaded at the block's first chunk, and one barrier in the
+// middle of each chunk is the only synchronisation. 2811 tokens, 6144 x 2048 Q4_K:
+// 183 us with both operands in LDS, 150 so (0.94 PFLOP/s of formed products); 2048 x
+// 6144 Q6_K: 245 and 195 us (1.09), where a large library product reaches 1.2; the
+// matrix cores are busy half of the time at 1.95 GHz.
+// For Q4_K the MFMAs, block scales and min terms of each
 // accumulator run in the order of MatMulMfmaKernel (the same bits for tiles
 // that are not split along K).
 typedef uint32_t U32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kPThreads = 512;
-constexpr int kPStage = 2 * kTileT * kRowStride;  // fp16 elements of one buffer's activation part
+constexpr int kPStage = kPlanes * kTileT * kChunk;  // fp16 elements of one chunk's activations
 
 template <uint32_t kType>
 struct PlanesCfg {
@@ -606,11 +611,20 @@ struct PlanesCfg {
   static constexpr int kOps = kQ4 ? 1 : 2;   // weight operands per column
   static constexpr int kNT = kQ4 ? 2 : 1;    // 32-row MFMA tiles per wave
   static constexpr int kTileR = 4 * 32 * kNT;
-  static constexpr int kBufHalfs = kPStage + kOps * kTileR * kRowStride;
 };
 
-// One thread per (row, block, 32-column run j = 2 kc + hf): the 32 operands
-// StageChunk<kQ4> builds for chunk kc, half hf, at the same chunk columns.
+// Weight planes in operand order: the 1 KB of operand o, rows 32 i .. + 31, columns
+// 16 k .. + 15 is what the 64 lanes of a wave hold for one matrix instruction, lane
+// after lane (row 32 i + lane % 32, columns 16 k + 8 (lane / 32) .. + 7), so that a
+// wave reads it as it lies, without LDS. Pieces of one i follow each other by k. The
+// rows past the last one in the last i are never written (nor are their products).
+__device__ __forceinline__ int64_t PlanePiece(int64_t row_groups, int op, int64_t row_group, int64_t cols, int64_t k16) {
+  return ((op * row_groups + row_group) * (cols / 16) + k16) * 512;
+}
+
+// One thread per (32 rows, block, row of them, 32-column run j = 2 kc + hf): the 32
+// operands StageChunk<kQ4> builds for chunk kc, half hf. A workgroup's 256 threads
+// have one block of 32 rows, so that the lines of the planes are written whole.
 struct PlanesArgs {
   const uint8_t* w;
   int64_t rows;
@@ -632,15 +646,21 @@ __device__ __forceinline__ void DecodeWeightUnit(const PlanesArgs& a, int64_t u)
   U32x4* __restrict__ mm = a.mm;
   constexpr bool kQ4 = kType == kGgmlQ4_K;
   constexpr int64_t kBB = kQ4 ? kQ4KBlockBytes : kQ6KBlockBytes;
-  if (u >= rows * nb * 8) return;
   const int j = static_cast<int>(u & 7);
-  const int64_t rb = u >> 3;  // row * nb + block
-  const int64_t r = rb / nb;
-  const int b = static_cast<int>(rb - r * nb);
+  const int li = static_cast<int>(u >> 3) & 31;
+  const int64_t group = (u >> 8) / nb;  // of 32 rows
+  const int b = static_cast<int>((u >> 8) - group * nb);
+  const int64_t r = 32 * group + li;
+  if (r >= rows) return;
+  const int64_t rb = r * nb + b;
   const int kc = j >> 1, hf = j & 1;
   const int64_t cols = static_cast<int64_t>(nb) * kQK_K;
+  const int64_t groups = (rows + 31) / 32;
   const uint8_t* blk = w + r * row_bytes + b * kBB;
-  _Float16* dst = planes + r * cols + static_cast<int64_t>(kQK_K) * b + kChunk * kc;
+  // column 16 s + 8 g of the chunk, operand op
+  const auto dst = [&](int op, int s, int g) {
+    return reinterpret_cast<F16x8*>(planes + PlanePiece(groups, op, group, cols, 16 * b + 4 * kc + s) + (32 * g + li) * 8);
+  };
   const StageRaw raw = kQ4 ? FetchStageQ4K(blk, kc, hf) : FetchStageQ6K(blk, kc, hf);
   if (kQ4) {
     const uint32_t s0 = raw.hdr.y, s1 = raw.hdr.z, s2 = raw.hdr.w;
@@ -652,8 +672,8 @@ __device__ __forceinline__ void DecodeWeightUnit(const PlanesArgs& a, int64_t u)
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
       const uint32_t bx = raw.q[2 * g], by = raw.q[2 * g + 1];
-      *reinterpret_cast<F16x8*>(dst + 16 * hf + 8 * g) = ScaledQ4(make_uint2(bx & 0x0F0F0F0Fu, by & 0x0F0F0F0Fu), fl);
-      *reinterpret_cast<F16x8*>(dst + 32 + 16 * hf + 8 * g) =
+      *dst(0, hf, g) = ScaledQ4(make_uint2(bx & 0x0F0F0F0Fu, by & 0x0F0F0F0Fu), fl);
+      *dst(0, 2 + hf, g) =
           ScaledQ4(make_uint2((bx >> 4) & 0x0F0F0F0Fu, (by >> 4) & 0x0F0F0F0Fu), fh);
     }
     if (j == 0) {
@@ -668,7 +688,6 @@ __device__ __forceinline__ void DecodeWeightUnit(const PlanesArgs& a, int64_t u)
       dd[rb] = make_float2(HalfF(raw.hdr.x & 0xFFFFu), HalfF(raw.hdr.x >> 16));
     }
   } else {
-    const int64_t plane = rows * cols;
     const int quarter = 2 * (kc & 1) + hf;
     const int nshift = quarter < 2 ? 0 : 4;
 #pragma unroll
@@ -689,8 +708,8 @@ __device__ __forceinline__ void DecodeWeightUnit(const PlanesArgs& a, int64_t u)
         wh[i] = a;
         wl[i] = static_cast<_Float16>(wf - static_cast<float>(a));
       }
-      *reinterpret_cast<F16x8*>(dst + 32 * hf + 8 * g) = wh;
-      *reinterpret_cast<F16x8*>(dst + plane + 32 * hf + 8 * g) = wl;
+      *dst(0, 2 * hf + (g >> 1), g & 1) = wh;
+      *dst(1, 2 * hf + (g >> 1), g & 1) = wl;
     }
     if (j == 0) dd[rb] = make_float2(HalfF(raw.hdr.x & 0xFFFFu), 0.0f);
   }
@@ -731,13 +750,14 @@ __global__ __launch_bounds__(kPThreads, 1) void MatMulMfmaPlanesKernel(
   constexpr bool kQ4 = C::kQ4;
   constexpr int kOps = C::kOps;
   constexpr int kNT = C::kNT;
-  __shared__ __attribute__((aligned(16))) _Float16 lds[2 * C::kBufHalfs];
+  // an array for each: a read waits only for the loads into its own array
+  __shared__ __attribute__((aligned(16))) _Float16 lds0[kPStage], lds1[kPStage], lds2[kPStage], lds3[kPStage];
   __shared__ float2 be_d[C::kTileR];                       // (d, dmin) of each row
   __shared__ U32x4 be_m[kQ4 ? C::kTileR : 1];              // Q4_K: m_j 2^6 of each row
   __shared__ U32x4 be_s[kQ4 ? kPlanes : 1][kQ4 ? kTileT : 1];  // Q4_K: run sums of each token
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 2;  // 64-token half of the tile
   const int wn = wave & 3;   // 32 kNT-row quarter of the tile
   const int li = lane & 31;
@@ -766,55 +786,51 @@ __global__ __launch_bounds__(kPThreads, 1) void MatMulMfmaPlanesKernel(
         part[mt][nt][i] = 0.0f;
       }
 
-  // staging map: 16-byte piece j of thread tid is row (tid >> 3) + 64 j' of
-  // its operand, segment tid & 7 of the chunk. Activations: j = 0..3 ->
-  // plane j >> 1, token rows 64 (j & 1) + tid >> 3 (clamped; a token past
-  // n_tokens reads a valid row whose outputs are never stored). Weights:
-  // j = 0..3 -> operand j / (4 / kOps), rows 64 (j % (4 / kOps)) + tid >> 3
-  // (clamped to the last row likewise).
-  // element offsets are 32-bit: the launcher checks that both operand
-  // images hold fewer than 2^31 elements
-  const int seg = tid & 7;
-  const int row8 = tid >> 3;
+  // Activations: a chunk is kPlanes x 128 rows of 128 bytes in LDS, 16-byte piece p of
+  // row t at p ^ (t / 2) % 8 (16 rows of a piece then lie in 16 different bank groups).
+  // Load j of wave w takes rows 64 j + 8 w + lane / 8, straight to LDS; the lanes'
+  // sources are chosen for the exchange. Tokens past n_tokens read a valid row whose
+  // outputs are never stored. Element offsets are 32-bit: the launcher checks that
+  // both operand images hold fewer than 2^31 elements.
   const int icols = static_cast<int>(cols);
-  U32x4 ra[4], rb[4];
-  int aoff[2];
+  uint32_t aoff[2];  // bytes
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
-    int64_t t = t0 + 64 * k + row8;
-    t = t < n_tokens ? t : n_tokens - 1;
-    aoff[k] = static_cast<int>(t) * icols + kQK_K * b0 + 8 * seg;
+    const int row = 64 * k + 8 * wave + (lane >> 3);
+    const int64_t t = t0 + row < n_tokens ? t0 + row : n_tokens - 1;
+    aoff[k] = 2u * static_cast<uint32_t>(static_cast<int>(t) * icols + kQK_K * b0 + 8 * ((lane & 7) ^ ((row >> 1) & 7)));
   }
-  constexpr int kRowsPerOp = 4 / kOps;  // 64-row groups per operand
-  int boff[kRowsPerOp];
+  __amdgpu_buffer_rsrc_t ars[kPlanes];
 #pragma unroll
-  for (int k = 0; k < kRowsPerOp; ++k) {
-    int64_t r = r0 + 64 * k + row8;
-    r = r < rows ? r : rows - 1;
-    boff[k] = static_cast<int>(r) * icols + kQK_K * b0 + 8 * seg;
-  }
-  const int iplane = static_cast<int>(plane_elems);
-  const int wplane = static_cast<int>(rows * cols);
-  const int lds_a = row8 * kRowStride + 8 * seg;
-  const int lds_b = kPStage + row8 * kRowStride + 8 * seg;
-
-#define RPG_PLANES_LOAD(c)                                                                                  \
-  do {                                                                                                      \
-    const int off_ = (c) * kChunk;                                                                          \
-    _Pragma("unroll") for (int j = 0; j < 4; ++j) ra[j] =                                                   \
-        *reinterpret_cast<const U32x4*>(planes + (aoff[j & 1] + (j >> 1) * iplane + off_));                 \
-    _Pragma("unroll") for (int j = 0; j < 4; ++j) rb[j] =                                                   \
-        *reinterpret_cast<const U32x4*>(wplanes + (boff[j % kRowsPerOp] + (j / kRowsPerOp) * wplane + off_)); \
-  } while (0)
-#define RPG_PLANES_STAGE(buf)                                                                               \
-  do {                                                                                                      \
-    _Float16* base_ = lds + (buf) * C::kBufHalfs;                                                           \
-    _Pragma("unroll") for (int j = 0; j < 4; ++j)                                                           \
-        *reinterpret_cast<U32x4*>(base_ + lds_a + ((j >> 1) * kTileT + 64 * (j & 1)) * kRowStride) = ra[j]; \
-    _Pragma("unroll") for (int j = 0; j < 4; ++j)                                                           \
-        *reinterpret_cast<U32x4*>(base_ + lds_b +                                                           \
-                                  ((j / kRowsPerOp) * C::kTileR + 64 * (j % kRowsPerOp)) * kRowStride) = rb[j]; \
-  } while (0)
+  for (int p = 0; p < kPlanes; ++p) ars[p] = dev::OutResource(const_cast<_Float16*>(planes + p * plane_elems), static_cast<uint32_t>(2 * plane_elems));
+  const auto load_a = [&](int c, _Float16* buf) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          ars[j >> 1], (__attribute__((address_space(3))) void*)(buf + ((j >> 1) * kTileT + 64 * (j & 1) + 8 * wave) * kChunk),
+          16, aoff[j & 1], 2 * kChunk * c, 0, 0);
+    }
+  };
+  // Weights: the wave's operands of K-step s of a chunk, from their planes to registers.
+  // Row groups past the last one read that one; their products are never stored.
+  const int64_t row_groups = (rows + 31) / 32;
+  uint32_t woff[kNT * kOps];  // bytes
+#pragma unroll
+  for (int nt = 0; nt < kNT; ++nt)
+#pragma unroll
+    for (int o = 0; o < kOps; ++o) {
+      const int64_t rg = r0 / 32 + kNT * wn + nt;
+      woff[nt * kOps + o] =
+          2u * static_cast<uint32_t>(PlanePiece(row_groups, o, rg < row_groups ? rg : row_groups - 1, cols, 16 * b0));
+    }
+  const __amdgpu_buffer_rsrc_t wrs =
+      dev::OutResource(const_cast<_Float16*>(wplanes), 2u * static_cast<uint32_t>(kOps * row_groups * 32 * cols));
+  F16x8 wf[4][kNT * kOps];
+  const auto load_w = [&](int c, int s) {
+#pragma unroll
+    for (int i = 0; i < kNT * kOps; ++i)
+      wf[s][i] = __builtin_bit_cast(F16x8, __builtin_amdgcn_raw_buffer_load_b128(wrs, 16 * lane, woff[i] + 1024 * (4 * c + s), 0));
+  };
 
   // Block-end values of the tile, through LDS (registers are the scarce
   // resource): per row (d, dmin) and m_j 2^6, per token and plane the
@@ -855,21 +871,16 @@ __global__ __launch_bounds__(kPThreads, 1) void MatMulMfmaPlanesKernel(
 
   // first: the block's first K-step, whose first product per accumulator
   // starts from zero (an exact sum, so no zeroing pass at the block end)
-  auto k_step = [&](int buf, int ks, bool first) {
-    const _Float16* xs = lds + buf * C::kBufHalfs;
-    const _Float16* ws = xs + kPStage;
-    const int kcol = 16 * ks + 8 * h;
-    F16x8 af[2][kPlanes], bf[kNT][kOps];
-#pragma unroll
-    for (int nt = 0; nt < kNT; ++nt)
-#pragma unroll
-      for (int o = 0; o < kOps; ++o)
-        bf[nt][o] = *reinterpret_cast<const F16x8*>(ws + (o * C::kTileR + 32 * kNT * wn + 32 * nt + li) * kRowStride + kcol);
+  const int a_lane = (64 * wm + li) * kChunk + 8 * (h ^ ((li >> 1) & 7));
+  F16x8 af[2][2][kPlanes];  // of this K-step and of the next one
+  auto read_a = [&](const _Float16* xs, int ks) {
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
       for (int p = 0; p < kPlanes; ++p)
-        af[mt][p] = *reinterpret_cast<const F16x8*>(xs + (p * kTileT + 64 * wm + 32 * mt + li) * kRowStride + kcol);
+        af[ks & 1][mt][p] = *reinterpret_cast<const F16x8*>(xs + (p * kTileT + 32 * mt) * kChunk + (a_lane ^ (16 * ks)));
+  };
+  auto k_step = [&](int ks, bool first) {
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
@@ -880,7 +891,7 @@ __global__ __launch_bounds__(kPThreads, 1) void MatMulMfmaPlanesKernel(
           for (int o = 0; o < kOps; ++o) {
             if (p == 1 && o == 1) continue;  // Q6_K x_lo w_lo: below 2^-22 |x w|, not formed
             const F32x16 zero = {};
-            part[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mt][p], bf[nt][o],
+            part[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[ks & 1][mt][p], wf[ks][nt * kOps + o],
                                                                   first && p == 0 && o == 0 ? zero : part[mt][nt], 0, 0, 0);
           }
   };
@@ -926,39 +937,54 @@ __global__ __launch_bounds__(kPThreads, 1) void MatMulMfmaPlanesKernel(
     }
   };
 
-  // The loads and LDS writes are unconditional (the last chunks re-stage the
-  // final chunk into the idle buffer): registers filled under a condition that
-  // spans iterations end up in scratch memory.
+  // Chunk c is in array c % 4. Each K-step first reads the next one's activations and
+  // then sends for the next chunk's weights in place of its own. In the middle of chunk
+  // c, behind the barrier that shows chunk c + 1 to be there and chunk c - 1 to be read,
+  // chunk c + 3 is sent for, to the array of c - 1: the waves go from chunk to chunk
+  // without waiting. The loads are unconditional (the last chunks load the final chunk
+  // again): registers filled under a condition that spans iterations end up in scratch
+  // memory.
   const int last = n_chunks - 1;
   fetch_block_end(b0);
-  RPG_PLANES_LOAD(0);
-  RPG_PLANES_STAGE(0);
-  RPG_PLANES_LOAD(last > 0 ? 1 : 0);
-  store_block_end();
-  __syncthreads();
-  for (int blk = 0; blk < n_blk; ++blk) {
-    // A block's end values are fetched at its first chunk, ahead of that
-    // chunk's staging loads (so the wait before the next LDS writes never
-    // waits for a load issued after them), and stored to LDS before the
-    // chunk's barrier; the previous block's end read them three barriers
-    // earlier.
-    if (blk > 0) fetch_block_end(b0 + blk);
+  load_a(0, lds0);
+  load_a(last > 0 ? 1 : 0, lds1);
+  load_a(last > 1 ? 2 : last, lds2);
 #pragma unroll
-    for (int kc = 0; kc < 4; ++kc) {  // chunk 4 blk + kc, in LDS buffer kc & 1
-      const int c = 4 * blk + kc;
-      k_step(kc & 1, 0, kc == 0);
-      RPG_PLANES_STAGE((kc & 1) ^ 1);
-      RPG_PLANES_LOAD(c + 2 < last ? c + 2 : last);
-      k_step(kc & 1, 1, false);
-      k_step(kc & 1, 2, false);
-      k_step(kc & 1, 3, false);
-      if (kc == 0 && blk > 0) store_block_end();
-      if (kc == 3) block_end();
-      __syncthreads();
+  for (int s = 0; s < 4; ++s) load_w(0, s);
+  store_block_end();
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  read_a(lds0, 0);
+  const auto chunk = [&](int blk, int kc, const _Float16* xs, const _Float16* xnext, _Float16* xlater) {
+    const int c = 4 * blk + kc;
+    const int cw = c < last ? c + 1 : last;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      read_a(s < 3 ? xs : xnext, (s + 1) & 3);
+      __builtin_amdgcn_sched_barrier(0);
+      k_step(s, kc == 0 && s == 0);
+      load_w(cw, s);
+      __builtin_amdgcn_sched_barrier(0);
+      if (s == 1) {
+        // 20 loads (or more, with a block's end values) are newer than chunk c + 1's
+        asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        load_a(c + 3 < last ? c + 3 : last, xlater);
+        if (kc == 0 && blk > 0) store_block_end();  // read in chunk 3 of the block, two barriers on
+      }
     }
+    if (kc == 3) block_end();
+  };
+  for (int blk = 0; blk < n_blk; ++blk) {
+    if (blk > 0) fetch_block_end(b0 + blk);
+    chunk(blk, 0, lds0, lds1, lds3);
+    chunk(blk, 1, lds1, lds2, lds0);
+    chunk(blk, 2, lds2, lds3, lds1);
+    chunk(blk, 3, lds3, lds0, lds2);
   }
-#undef RPG_PLANES_LOAD
-#undef RPG_PLANES_STAGE
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last chunk's repeated loads: nothing lands in LDS after the end
 
   if (split) {
     float* dst = partial + static_cast<int64_t>(g - dp_tiles) * kTileT * C::kTileR;
@@ -1138,7 +1164,7 @@ void LaunchPendingSplit(const SplitActivations& sa) {
 // The weight decode of one row slice, with a pending split in the same launch.
 template <uint32_t kType>
 void LaunchDecode(const PlanesArgs& pa, const SplitActivations& sa) {
-  const int64_t units = pa.rows * pa.nb * 8;
+  const int64_t units = (pa.rows + 31) / 32 * 32 * pa.nb * 8;
   const unsigned decode_wgs = GridFor(units, kThreads);
   if (!sa.pending) {
     Launch(kType == kGgmlQ4_K ? "DecodeWeightPlanesQ4KKernel" : "DecodeWeightPlanesQ6KKernel",
@@ -1166,7 +1192,7 @@ void LaunchPlanesRows(const uint8_t* w, int64_t rows, int64_t row_bytes, int32_t
                       float* out, int64_t ldo) {
   using C = PlanesCfg<kType>;
   const int64_t cols = static_cast<int64_t>(nb) * kQK_K;
-  const size_t plane_bytes = static_cast<size_t>(C::kOps) * rows * cols * sizeof(_Float16);
+  const size_t plane_bytes = static_cast<size_t>(C::kOps) * ((rows + 31) / 32 * 32) * cols * sizeof(_Float16);
   const size_t dd_off = (plane_bytes + 255) / 256 * 256;
   const size_t mm_off = dd_off + (static_cast<size_t>(rows) * nb * sizeof(float2) + 255) / 256 * 256;
   const size_t bytes = mm_off + static_cast<size_t>(rows) * nb * sizeof(U32x4);
