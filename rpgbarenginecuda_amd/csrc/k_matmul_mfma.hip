@@ -1017,26 +1017,42 @@ __global__ __launch_bounds__(kPThreads, 1) void MatMulMfmaPlanesKernel(
   }
 }
 
-// out = the sum over slices, in order, of the split tiles' partial tiles.
-template <int kTileRows>
-__global__ __launch_bounds__(kThreads) void MatMulPlanesReduceKernel(const float* __restrict__ partial,
-                                                                      int64_t split_tiles, int32_t splits,
+// out = the sum over slices, in order, of the split tiles' partial tiles: a workgroup
+// 1024 elements of one of them, four rows of a token in each thread. It moves
+// data and nothing else, so the indexing is 32-bit and per workgroup, and each thread
+// has the 16 bytes of four slices in flight (one element per thread, each with its own
+// 64-bit divisions: 14.4 us for five slices of 700 tokens on 4096 x 2560, 10.8 so). kWide: out's rows of
+// four may be stored whole.
+template <int kTileRows, bool kWide>
+__global__ __launch_bounds__(kThreads) void MatMulPlanesReduceKernel(const float* __restrict__ partial, int32_t splits,
                                                                       int32_t row_tiles, int32_t dp_tiles,
                                                                       int64_t n_tokens, int64_t rows,
                                                                       float* __restrict__ out, int64_t ldo) {
-  constexpr int64_t kTileElems = static_cast<int64_t>(kTileT) * kTileRows;
-  const int64_t e = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-  if (e >= split_tiles * kTileElems) return;
-  const int64_t st = e / kTileElems;
-  const int64_t le = e - st * kTileElems;
-  const int64_t tile = dp_tiles + st;
-  const int64_t tok = (tile / row_tiles) * kTileT + le / kTileRows;
-  const int64_t row = (tile % row_tiles) * kTileRows + le % kTileRows;
+  constexpr int kTileElems = kTileT * kTileRows;
+  constexpr uint32_t kParts = kTileElems / (4 * kThreads);
+  const int st = static_cast<int>(blockIdx.x / kParts);
+  const int le = 4 * static_cast<int>(blockIdx.x % kParts * kThreads + threadIdx.x);
+  const int tile = dp_tiles + st;
+  const int tile_t = tile / row_tiles;
+  const int64_t tok = static_cast<int64_t>(tile_t) * kTileT + le / kTileRows;
+  const int64_t row = static_cast<int64_t>(tile - tile_t * row_tiles) * kTileRows + le % kTileRows;
   if (tok >= n_tokens || row >= rows) return;
-  const float* p = partial + st * splits * kTileElems + le;
-  float v = p[0];
-  for (int32_t z = 1; z < splits; ++z) v += p[z * kTileElems];
-  out[tok * ldo + row] = v;
+  const float4* p = reinterpret_cast<const float4*>(partial + static_cast<int64_t>(st) * splits * kTileElems + le);
+  float4 v = p[0];
+#pragma unroll 4
+  for (int32_t z = 1; z < splits; ++z) {
+    const float4 w = p[static_cast<int64_t>(z) * (kTileElems / 4)];
+    v = make_float4(v.x + w.x, v.y + w.y, v.z + w.z, v.w + w.w);
+  }
+  float* o = out + tok * ldo + row;
+  if (kWide) {
+    *reinterpret_cast<float4*>(o) = v;
+    return;
+  }
+  o[0] = v.x;
+  if (row + 1 < rows) o[1] = v.y;
+  if (row + 2 < rows) o[2] = v.z;
+  if (row + 3 < rows) o[3] = v.w;
 }
 
 }  // namespace
@@ -1209,11 +1225,16 @@ void LaunchPlanesRows(const uint8_t* w, int64_t rows, int64_t row_bytes, int32_t
   // One workgroup per CU, so a grid runs in rounds of kCUs workgroups. Plans:
   // whole rounds of tiles unsplit and the tiles left over split along K to
   // fill the last round (dp = the whole rounds), or every tile split alike
-  // (dp = 0). Each is priced as rounds x blocks per workgroup x the time of
-  // one block of one tile, plus the reduce (slices + 1 passes over the split
-  // tiles at ~4 TB/s); the cheapest wins.
+  // (dp = 0). Each is priced as rounds x (the first loads and the tile's stores, and
+  // blocks per workgroup x the time of one block of one tile), plus the reduce (its
+  // launch, and slices + 1 passes over the split tiles at 8 TB/s from the caches); the
+  // cheapest wins. Measured at 700 tokens: 1024, 4096 and 2560 rows of Q4_K in one
+  // round of 1 block, two of 2 and one of 4 take 22, 54 and 42 us, their reduces 5.9,
+  // 10.9 and 6.2; without the rounds' price 4096 x 2560 took two rounds and 65 us in
+  // all, and takes one and 48 with it.
   constexpr int64_t kCUs = 256;
-  constexpr double kBlockUs = C::kQ4 ? 10.0 : 6.6;  // measured, 2811 tokens
+  constexpr double kRoundUs = 10.5;
+  constexpr double kBlockUs = C::kQ4 ? 6.7 : 4.5;
   const double tile_bytes = 4.0 * kTileT * C::kTileR;
   int64_t best_dp = tiles;
   int32_t best_splits = 1, best_bps = nb;
@@ -1226,8 +1247,9 @@ void LaunchPlanesRows(const uint8_t* w, int64_t rows, int64_t row_bytes, int32_t
       const int32_t slices = (nb + b - 1) / b;
       if (rest == 0 && slices > 1) break;
       const int64_t rounds_rest = (rest * slices + kCUs - 1) / kCUs;
-      const double us = static_cast<double>(dp / kCUs) * nb * kBlockUs + static_cast<double>(rounds_rest) * b * kBlockUs +
-                        (slices > 1 ? (slices + 1) * static_cast<double>(rest) * tile_bytes / 4e6 : 0.0);
+      const double us = static_cast<double>(dp / kCUs) * (kRoundUs + nb * kBlockUs) +
+                        static_cast<double>(rounds_rest) * (kRoundUs + b * kBlockUs) +
+                        (slices > 1 ? 2.0 + (slices + 1) * static_cast<double>(rest) * tile_bytes / 8e6 : 0.0);
       if (best == 0.0 || us < best) {
         best = us;
         best_dp = slices > 1 ? dp : tiles;
@@ -1249,10 +1271,12 @@ void LaunchPlanesRows(const uint8_t* w, int64_t rows, int64_t row_bytes, int32_t
          static_cast<const _Float16*>(sa.planes), static_cast<const _Float16*>(sa.sums), sa.sum_stride, sa.inv_scale,
          sa.n_tokens, static_cast<int32_t>(gx), static_cast<int32_t>(best_dp), best_splits, best_bps, out, ldo, partial);
   if (split_tiles > 0) {
-    const int64_t elems = split_tiles * kTileT * C::kTileR;
-    Launch("MatMulPlanesReduceKernel", MatMulPlanesReduceKernel<C::kTileR>, dim3(GridFor(elems, kThreads)),
-           dim3(kThreads), static_cast<const float*>(partial), split_tiles, best_splits, static_cast<int32_t>(gx),
-           static_cast<int32_t>(best_dp), sa.n_tokens, rows, out, ldo);
+    const bool wide = rows % 4 == 0 && ldo % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 15u) == 0;
+    Launch("MatMulPlanesReduceKernel",
+           wide ? MatMulPlanesReduceKernel<C::kTileR, true> : MatMulPlanesReduceKernel<C::kTileR, false>,
+           dim3(static_cast<unsigned>(split_tiles * (kTileT * C::kTileR / (4 * kThreads)))), dim3(kThreads),
+           static_cast<const float*>(partial), best_splits, static_cast<int32_t>(gx), static_cast<int32_t>(best_dp),
+           sa.n_tokens, rows, out, ldo);
   }
 }
 
