@@ -31,6 +31,7 @@
 // workgroups share a CU and cover each other's barriers and LDS latency.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 
@@ -1141,11 +1142,11 @@ void* EnsureWeightPlanes(size_t bytes) {
   return b.ptr;
 }
 
-// Decoded planes are used for grids of many tiles (from kPlanesMinTokens
-// tokens). A matrix whose planes exceed kPlanesMaxBytes (a 151936-row output
+// Decoded planes are used for grids of many tiles: from kPlanesMinTokens tokens, and
+// from kPlanesFewTokens where they are estimated to be the faster. A matrix whose planes exceed kPlanesMaxBytes (a 151936-row output
 // projection) is decoded and multiplied in row slices that fit, each writing
 // its columns of OUT.
-constexpr int64_t kPlanesMinTokens = 512;
+constexpr int64_t kPlanesMinTokens = 512, kPlanesFewTokens = 385;
 constexpr size_t kPlanesMaxBytes = size_t{64} << 20;
 
 // OUT[:, 0 : rows) with row stride ldo for the `rows` weight rows at w.
@@ -1203,42 +1204,27 @@ void LaunchDecode(const PlanesArgs& pa, const SplitActivations& sa) {
   }
 }
 
-template <uint32_t kType>
-void LaunchPlanesRows(const uint8_t* w, int64_t rows, int64_t row_bytes, int32_t nb, const SplitActivations& sa,
-                      float* out, int64_t ldo) {
-  using C = PlanesCfg<kType>;
-  const int64_t cols = static_cast<int64_t>(nb) * kQK_K;
-  const size_t plane_bytes = static_cast<size_t>(C::kOps) * ((rows + 31) / 32 * 32) * cols * sizeof(_Float16);
-  const size_t dd_off = (plane_bytes + 255) / 256 * 256;
-  const size_t mm_off = dd_off + (static_cast<size_t>(rows) * nb * sizeof(float2) + 255) / 256 * 256;
-  const size_t bytes = mm_off + static_cast<size_t>(rows) * nb * sizeof(U32x4);
-  uint8_t* base = static_cast<uint8_t*>(EnsureWeightPlanes(bytes));
-  _Float16* wplanes = reinterpret_cast<_Float16*>(base);
-  float2* dd = reinterpret_cast<float2*>(base + dd_off);
-  U32x4* mm = reinterpret_cast<U32x4*>(base + mm_off);
-  LaunchDecode<kType>(PlanesArgs{w, rows, row_bytes, nb, wplanes, dd, mm}, sa);
-
-  const int64_t gy = (sa.n_tokens + kTileT - 1) / kTileT;
-  const int64_t gx = (rows + C::kTileR - 1) / C::kTileR;
-  const int64_t tiles = gx * gy;
-  RPG_CHECK(tiles * 8 <= 0x7FFFFFFF, "matmul grid too large: %lld tiles", static_cast<long long>(tiles));
-  // One workgroup per CU, so a grid runs in rounds of kCUs workgroups. Plans:
-  // whole rounds of tiles unsplit and the tiles left over split along K to
-  // fill the last round (dp = the whole rounds), or every tile split alike
-  // (dp = 0). Each is priced as rounds x (the first loads and the tile's stores, and
-  // blocks per workgroup x the time of one block of one tile), plus the reduce (its
-  // launch, and slices + 1 passes over the split tiles at 8 TB/s from the caches); the
-  // cheapest wins. Measured at 700 tokens: 1024, 4096 and 2560 rows of Q4_K in one
-  // round of 1 block, two of 2 and one of 4 take 22, 54 and 42 us, their reduces 5.9,
-  // 10.9 and 6.2; without the rounds' price 4096 x 2560 took two rounds and 65 us in
-  // all, and takes one and 48 with it.
+// One workgroup per CU, so a grid runs in rounds of kCUs workgroups. Plans:
+// whole rounds of tiles unsplit and the tiles left over split along K to
+// fill the last round (dp = the whole rounds), or every tile split alike
+// (dp = 0). Each is priced as rounds x (the first loads and the tile's stores, and
+// blocks per workgroup x the time of one block of one tile), plus the reduce (its
+// launch, and slices + 1 passes over the split tiles at 8 TB/s from the caches); the
+// cheapest wins. Measured at 700 tokens: 1024, 4096 and 2560 rows of Q4_K in one
+// round of 1 block, two of 2 and one of 4 take 22, 54 and 42 us, their reduces 5.9,
+// 10.9 and 6.2; without the rounds' price 4096 x 2560 took two rounds and 65 us in
+// all, and takes one and 48 with it.
+struct PlanesPlan {
+  int64_t dp = 0;
+  int32_t splits = 1, bps = 0;
+  double us = 0.0;
+};
+PlanesPlan PlanFor(bool q4, int64_t tiles, int32_t nb) {
   constexpr int64_t kCUs = 256;
   constexpr double kRoundUs = 10.5;
-  constexpr double kBlockUs = C::kQ4 ? 6.7 : 4.5;
-  const double tile_bytes = 4.0 * kTileT * C::kTileR;
-  int64_t best_dp = tiles;
-  int32_t best_splits = 1, best_bps = nb;
-  double best = 0.0;
+  const double block_us = q4 ? 6.7 : 4.5;
+  const double tile_bytes = 4.0 * kTileT * (q4 ? PlanesCfg<kGgmlQ4_K>::kTileR : PlanesCfg<kGgmlQ6_K>::kTileR);
+  PlanesPlan best;
   for (int plan = 0; plan < 2; ++plan) {
     const int64_t dp = plan == 0 ? tiles / kCUs * kCUs : 0;
     const int64_t rest = tiles - dp;
@@ -1247,17 +1233,72 @@ void LaunchPlanesRows(const uint8_t* w, int64_t rows, int64_t row_bytes, int32_t
       const int32_t slices = (nb + b - 1) / b;
       if (rest == 0 && slices > 1) break;
       const int64_t rounds_rest = (rest * slices + kCUs - 1) / kCUs;
-      const double us = static_cast<double>(dp / kCUs) * (kRoundUs + nb * kBlockUs) +
-                        static_cast<double>(rounds_rest) * (kRoundUs + b * kBlockUs) +
+      const double us = static_cast<double>(dp / kCUs) * (kRoundUs + nb * block_us) +
+                        static_cast<double>(rounds_rest) * (kRoundUs + b * block_us) +
                         (slices > 1 ? 2.0 + (slices + 1) * static_cast<double>(rest) * tile_bytes / 8e6 : 0.0);
-      if (best == 0.0 || us < best) {
-        best = us;
-        best_dp = slices > 1 ? dp : tiles;
-        best_splits = slices;
-        best_bps = b;
-      }
+      if (best.us == 0.0 || us < best.us) best = PlanesPlan{slices > 1 ? dp : tiles, slices, b, us};
     }
   }
+  return best;
+}
+
+// The weight-plane buffer of one row slice: planes, then (d, dmin), then m.
+struct PlanesLayout {
+  size_t dd, mm, bytes;
+  PlanesLayout(bool q4, int64_t rows, int32_t nb) {
+    const size_t planes = static_cast<size_t>(q4 ? 1 : 2) * ((rows + 31) / 32 * 32) * nb * kQK_K * sizeof(_Float16);
+    dd = (planes + 255) / 256 * 256;
+    mm = dd + (static_cast<size_t>(rows) * nb * sizeof(float2) + 255) / 256 * 256;
+    bytes = mm + static_cast<size_t>(rows) * nb * sizeof(U32x4);
+  }
+};
+
+// Rows decoded and multiplied at a time.
+int64_t PlanesSlice(bool q4, int32_t nb) {
+  const int64_t tile = q4 ? PlanesCfg<kGgmlQ4_K>::kTileR : PlanesCfg<kGgmlQ6_K>::kTileR;
+  const int64_t row_plane_bytes = static_cast<int64_t>(q4 ? 1 : 2) * nb * kQK_K * sizeof(_Float16);
+  const int64_t slice = static_cast<int64_t>(kPlanesMaxBytes) / row_plane_bytes / tile * tile;
+  return slice < tile ? tile : slice;
+}
+
+// A whole matrix on the planes: its time (per slice, the decode's launch and its bytes,
+// the GEMM's launch and plan), and the buffers that it takes.
+struct PlanesNeed {
+  double us = 0.0;
+  size_t weights = 0, partials = 0;
+  PlanesNeed(bool q4, int64_t rows, int32_t nb, int64_t n_tokens) {
+    const int64_t tile = q4 ? PlanesCfg<kGgmlQ4_K>::kTileR : PlanesCfg<kGgmlQ6_K>::kTileR;
+    const int64_t slice = PlanesSlice(q4, nb);
+    for (int64_t r = 0; r < rows; r += slice) {
+      const int64_t n = rows - r < slice ? rows - r : slice;
+      const int64_t tiles = (n_tokens + kTileT - 1) / kTileT * ((n + tile - 1) / tile);
+      const PlanesLayout lay(q4, n, nb);
+      const PlanesPlan plan = PlanFor(q4, tiles, nb);
+      us += 4.5 + static_cast<double>(lay.bytes) / 4e6 + 4.0 + plan.us;
+      weights = std::max(weights, lay.bytes);
+      partials = std::max(partials, static_cast<size_t>(tiles - plan.dp) * plan.splits * kTileT * tile * sizeof(float));
+    }
+  }
+};
+
+template <uint32_t kType>
+void LaunchPlanesRows(const uint8_t* w, int64_t rows, int64_t row_bytes, int32_t nb, const SplitActivations& sa,
+                      float* out, int64_t ldo) {
+  using C = PlanesCfg<kType>;
+  const PlanesLayout lay(C::kQ4, rows, nb);
+  uint8_t* base = static_cast<uint8_t*>(EnsureWeightPlanes(lay.bytes));
+  _Float16* wplanes = reinterpret_cast<_Float16*>(base);
+  float2* dd = reinterpret_cast<float2*>(base + lay.dd);
+  U32x4* mm = reinterpret_cast<U32x4*>(base + lay.mm);
+  LaunchDecode<kType>(PlanesArgs{w, rows, row_bytes, nb, wplanes, dd, mm}, sa);
+
+  const int64_t gy = (sa.n_tokens + kTileT - 1) / kTileT;
+  const int64_t gx = (rows + C::kTileR - 1) / C::kTileR;
+  const int64_t tiles = gx * gy;
+  RPG_CHECK(tiles * 8 <= 0x7FFFFFFF, "matmul grid too large: %lld tiles", static_cast<long long>(tiles));
+  const PlanesPlan plan = PlanFor(C::kQ4, tiles, nb);
+  const int64_t best_dp = plan.dp;
+  const int32_t best_splits = plan.splits, best_bps = plan.bps;
   const int64_t split_tiles = tiles - best_dp;
   float* partial = nullptr;
   if (split_tiles > 0) {
@@ -1283,17 +1324,35 @@ void LaunchPlanesRows(const uint8_t* w, int64_t rows, int64_t row_bytes, int32_t
 template <uint32_t kType>
 void LaunchPlanes(const uint8_t* w, int64_t rows, int64_t row_bytes, int32_t nb, const SplitActivations& sa,
                   float* out) {
-  using C = PlanesCfg<kType>;
-  const int64_t row_plane_bytes = static_cast<int64_t>(C::kOps) * nb * kQK_K * sizeof(_Float16);
-  int64_t slice = static_cast<int64_t>(kPlanesMaxBytes) / row_plane_bytes / C::kTileR * C::kTileR;
-  if (slice < C::kTileR) slice = C::kTileR;
+  const int64_t slice = PlanesSlice(kType == kGgmlQ4_K, nb);
   for (int64_t r = 0; r < rows; r += slice) {
     const int64_t n = rows - r < slice ? rows - r : slice;
     LaunchPlanesRows<kType>(w + r * row_bytes, n, row_bytes, nb, sa, out + r, rows);
   }
 }
 
+bool Holds(SplitBuffer& b, size_t bytes) {
+  std::lock_guard<std::mutex> lock(b.mu);
+  return b.bytes >= bytes;
+}
+
 }  // namespace
+
+// From four token tiles on: 9728 x 2560 Q4_K at 448 tokens 92 us on the planes and 105 on
+// the GEMM below, 2560 x 9728 Q6_K (two slices) 130 and 148. With three the decode pass
+// is too much of it (72 and 76 us at 333 tokens from caches, but 4% slower with weights
+// that come from memory).
+double PlanesUs(bool q6, int64_t rows, int32_t nb, int64_t n_tokens) {
+  return n_tokens < kPlanesFewTokens ? HUGE_VAL : PlanesNeed(!q6, rows, nb, n_tokens).us;
+}
+
+// The GEMM that decodes per 128-token tile: 20 us, more for a long K, and about 280
+// useful TFLOP/s (1024 x 2048 Q4_K: 24.5 us at 128 tokens, 29 at 448; 2560 x 9728 Q6_K:
+// 75 and 149).
+double MfmaUs(int64_t rows, int32_t nb, int64_t n_tokens) {
+  const double mega = static_cast<double>(rows) * 256e-6 * nb;  // weights, in millions
+  return 20.0 + 0.02 * nb * nb + 2.0 * static_cast<double>((n_tokens + 127) / 128 * 128) * mega / 280.0;
+}
 
 SplitActivations SplitForMfma(const float* x, int64_t n_tokens, int64_t cols) {
   RPG_CHECK(n_tokens > 0 && cols > 0 && cols % 32 == 0, "invalid activation split [%lld, %lld]",
@@ -1334,7 +1393,16 @@ void LaunchMatMulMfmaSplit(uint32_t type, const uint8_t* w, int64_t rows, int64_
             static_cast<long long>(sa.cols), static_cast<long long>(nb) * kQK_K);
   // (the planes kernel indexes both operand images with 32-bit offsets;
   // the weight slices stay within kPlanesMaxBytes)
-  if (sa.n_tokens >= kPlanesMinTokens && kPlanes * sa.n_tokens * sa.cols < (int64_t{1} << 31)) {
+  bool on_planes = kPlanes * sa.n_tokens * sa.cols < (int64_t{1} << 31);
+  if (on_planes && sa.n_tokens < kPlanesMinTokens) {
+    on_planes = sa.n_tokens >= kPlanesFewTokens &&
+                PlanesUs(type == kGgmlQ6_K, rows, nb, sa.n_tokens) < MfmaUs(rows, nb, sa.n_tokens);
+    if (on_planes && StreamIsCapturing()) {  // nothing may be allocated: only if the shape ran before
+      const PlanesNeed need(type == kGgmlQ4_K, rows, nb, sa.n_tokens);
+      on_planes = Holds(WeightPlanes(), need.weights) && Holds(PartialTiles(), need.partials);
+    }
+  }
+  if (on_planes) {
     if (type == kGgmlQ4_K) {
       LaunchPlanes<kGgmlQ4_K>(w, rows, row_bytes, nb, sa, out);
     } else {

@@ -37,6 +37,7 @@
 // (22 instead of 16 us for gate / up) were the largest costs taken out on the way.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "dev_util.h"
@@ -793,10 +794,8 @@ bool MatMulSmallWins(const SmallMat& m, int32_t nb, int64_t n_tokens) {
   // (2048 x 2048 Q4_K: 4.8 us at 2 tokens, 11.4 at 8, against 6.7 here; 2048 x 6144
   // Q6_K: 8.5 and 18.9 against 15).
   if (n_tokens < 32) return us <= 1.1 * (2.4 + (m.q6 ? 0.17 : 0.26) * static_cast<double>(n_tokens) * mega);
-  // The GEMM that decodes per 128-token tile: 20 us, more for a long K, and about 280
-  // useful TFLOP/s (1024 x 2048 Q4_K: 24.5 us at 128 tokens, 29 at 448; 2560 x 9728
-  // Q6_K: 75 and 149). Within a tenth of it the estimate above is the high one.
-  return us <= 1.1 * (20.0 + 0.02 * nb * nb + 2.0 * static_cast<double>((n_tokens + 127) / 128 * 128) * mega / 280.0);
+  // The prefill kernels. Within a tenth of them the estimate above is the high one.
+  return us <= 1.1 * std::min(MfmaUs(m.rows, nb, n_tokens), PlanesUs(m.q6, m.rows, nb, n_tokens));
 }
 
 void LaunchMatMulSmall(const SmallMat* mats, int32_t n_mats, int32_t nb, const float* x, int64_t n_tokens) {

@@ -37,6 +37,11 @@ void LaunchMatMulMfmaSplit(uint32_t type, const uint8_t* w, int64_t rows, int64_
 void LaunchMatMulMfma(uint32_t type, const uint8_t* w, int64_t rows, int64_t row_bytes, int32_t nb, const float* x,
                       int64_t cols, int64_t n_tokens, float* out);
 
+// Estimated times of a prefill matmul: on decoded weight planes (infinite below the
+// tokens that they are used for), and on the GEMM that decodes as it goes.
+double PlanesUs(bool q6, int64_t rows, int32_t nb, int64_t n_tokens);
+double MfmaUs(int64_t rows, int32_t nb, int64_t n_tokens);
+
 // A library-owned buffer of at least `bytes` for the partial results of K slices
 // (valid until the next split launch on the engine stream), and the launch that
 // sums them: out[e] = sum over z < splits of partial[z elems + e], in that order.

@@ -1,4 +1,5 @@
-"""The matmul on decoded weight planes (512 tokens and more): ragged row groups, row and
+"""The matmul on decoded weight planes (512 tokens and more, and fewer on large
+matrices): ragged row groups, row and
 token tiles, one block to several, against the float64 oracle within the bound of
 tests/test_gpu_matmul.py."""
 from __future__ import annotations
@@ -16,7 +17,7 @@ Q4, Q6 = 12, 14
 
 @pytest.mark.parametrize("t", [Q4, Q6])
 @pytest.mark.parametrize("rows,cols,n", [(1, 256, 512), (31, 768, 513), (33, 512, 640), (129, 1280, 700), (257, 2048, 641),
-                                         (300, 2560, 1025)])
+                                         (300, 2560, 1025), (9700, 2560, 385), (2560, 9728, 448)])
 def test_planes_matmul_vs_f64(gpu, ora, t, rows, cols, n):
     import torch
 
