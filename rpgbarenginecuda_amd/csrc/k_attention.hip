@@ -871,11 +871,16 @@ __device__ __forceinline__ F16x4 VTr(const _Float16* lds_ptr) {
   return __builtin_bit_cast(F16x4, v);
 }
 
-// 16 bytes per lane from global memory to LDS: lane i's at base + 16 i. The caller
-// waits (vmcnt) before it reads them.
-__device__ __forceinline__ void LoadToLds(const uint16_t* from, _Float16* base) {
-  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(from),
-                                   (__attribute__((address_space(3))) void*)(base), 16, 0, 0);
+// The rows of a block of `keys` cache rows as a buffer, and 16 bytes per lane from it to
+// LDS: lane i's at base + 16 i. The caller waits (vmcnt) before it reads them. (Buffer
+// loads and not global ones: after a global load to LDS the compiler lets no LDS read
+// wait for less than all of them.)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t CacheRows(const uint16_t* rows, int keys) {
+  return dev::OutResource(const_cast<uint16_t*>(rows), static_cast<uint32_t>(2 * kD * keys));
+}
+__device__ __forceinline__ void LoadToLds(__amdgpu_buffer_rsrc_t rows, uint32_t byte_off, _Float16* base) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, (__attribute__((address_space(3))) void*)(base), 16,
+                                           static_cast<int>(byte_off), 0, 0, 0);
 }
 
 // x as two fp16 terms, *h = fp16(x) and *l = fp16(x - h) (the difference is
@@ -996,14 +1001,22 @@ __device__ __forceinline__ void FaScores(const KOperand& k, const F16x8 (&qb)[2]
     for (int mt = 0; mt < kTiles; ++mt) st[mt] += sh[mt];
     return;
   }
+  F16x8 a[2][kTiles];  // of this step and of the next one, read ahead
+#pragma unroll
+  for (int mt = 0; mt < kTiles; ++mt) a[0][mt] = k(mt, 0);
 #pragma unroll
   for (int s = 0; s < 8; ++s) {
+    if (s < 7) {
 #pragma unroll
-    for (int mt = 0; mt < kTiles; ++mt) {
-      const F16x8 a = k(mt, s);
-      st[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qb[1][s], st[mt], 0, 0, 0);
-      st[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qb[0][s], st[mt], 0, 0, 0);
+      for (int mt = 0; mt < kTiles; ++mt) a[(s + 1) & 1][mt] = k(mt, s + 1);
     }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 1; t >= 0; --t)
+#pragma unroll
+      for (int mt = 0; mt < kTiles; ++mt)
+        st[mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[s & 1][mt], qb[t][s], st[mt], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
   }
 }
 
@@ -1091,15 +1104,18 @@ __device__ __forceinline__ void FaAttend(const VOperand& v, F32x16 (&st)[kTiles]
     }
     return;
   }
+  F16x8 a[2] = {v(0, 0), F16x8{}};  // this product's and the next one's, read ahead
 #pragma unroll
   for (int ks = 0; ks < 2 * kTiles; ++ks) {
     F16x8 ph, pl;
     split(ks, &ph, &pl);
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) {
-      const F16x8 a = v(ks, dt);
-      o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pl, o[dt], 0, 0, 0);
-      o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, ph, o[dt], 0, 0, 0);
+      if (ks + 1 < 2 * kTiles || dt < 3) a[(dt + 1) & 1] = v(dt < 3 ? ks : ks + 1, (dt + 1) & 3);
+      __builtin_amdgcn_sched_barrier(0x2 | 0x4);
+      o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[dt & 1], pl, o[dt], 0, 0, 0);
+      o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[dt & 1], ph, o[dt], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0x2 | 0x4);
     }
   }
 }
@@ -1132,7 +1148,7 @@ __global__ __launch_bounds__(256, 2) void AttnPrefillMfmaKernel(
   __shared__ __attribute__((aligned(16))) _Float16 ks0[kFaKeys * kD], ks1[kFaKeys * kD];
   __shared__ __attribute__((aligned(16))) _Float16 vs0[kFaKeys * kD], vs1[kFaKeys * kD];
   const int lane = threadIdx.x & 63;
-  const int wv = threadIdx.x >> 6;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int hf = lane >> 5;    // which half of the keys / dims this lane holds
   const int col = lane & 31;   // the lane's query within the wave
   const int32_t pair = static_cast<int32_t>(blockIdx.x) / n_heads;
@@ -1188,16 +1204,19 @@ __global__ __launch_bounds__(256, 2) void AttnPrefillMfmaKernel(
   const int kpiece = 8 * ((lane & 15) ^ (4 * wv + lrow));
   const int vpiece = 8 * ((lane & 15) ^ (4 * lrow));
   const auto stage = [&](int64_t kb, _Float16* kto, _Float16* vto) {
+    const __amdgpu_buffer_rsrc_t krows = CacheRows(kbase + kb * kD, kFaKeys);
+    const __amdgpu_buffer_rsrc_t vrows = CacheRows(vbase + kb * kD, kFaKeys);
+    const int visible = static_cast<int>(last_key - kb < kFaKeys ? last_key - kb : kFaKeys);
 #pragma unroll
     for (int j = 0; j < kFaKeys / 16; ++j) {
-      const int row = 16 * j + 4 * wv;
-      const int64_t key = kb + row + lrow < last_key ? kb + row + lrow : last_key;
+      const int to = (16 * j + 4 * wv) * kD;
+      const int row = 16 * j + 4 * wv + lrow < visible ? 16 * j + 4 * wv + lrow : visible;
       if constexpr (kDirect) {
-        LoadToLds(kbase + key * kD + kpiece, kto + row * kD);
-        LoadToLds(vbase + key * kD + vpiece, vto + row * kD);
+        LoadToLds(krows, 2 * (row * kD + kpiece), kto + to);
+        LoadToLds(vrows, 2 * (row * kD + vpiece), vto + to);
       } else {
-        *reinterpret_cast<uint4*>(kto + row * kD + 8 * lane) = *reinterpret_cast<const uint4*>(kbase + key * kD + kpiece);
-        *reinterpret_cast<uint4*>(vto + row * kD + 8 * lane) = *reinterpret_cast<const uint4*>(vbase + key * kD + vpiece);
+        *reinterpret_cast<uint4*>(kto + to + 8 * lane) = *reinterpret_cast<const uint4*>(kbase + (kb + row) * kD + kpiece);
+        *reinterpret_cast<uint4*>(vto + to + 8 * lane) = *reinterpret_cast<const uint4*>(vbase + (kb + row) * kD + vpiece);
       }
     }
   };
@@ -1433,11 +1452,12 @@ __global__ __launch_bounds__(64 * kTurnWaves, 1) void AttnTurnKernel(
   const uint16_t* const vbase = vc + kh * max_seq * kD;
   const uint32_t lrow = static_cast<uint32_t>(lane) >> 4;
   const auto load = [&](const uint16_t* base, int64_t kb, uint32_t piece, uint32_t turn, _Float16* to) {
+    const __amdgpu_buffer_rsrc_t rows = CacheRows(base + kb * kD, kTurnKeys);
     const uint32_t visible = static_cast<uint32_t>(last_key - kb < kTurnKeys ? last_key - kb : kTurnKeys);
 #pragma unroll
     for (uint32_t j = 0; j < kTurnKeys / 4; ++j) {
       const uint32_t row = 4 * j + lrow < visible ? 4 * j + lrow : visible;
-      LoadToLds(base + kb * kD + (row * kD + 8 * (piece ^ (turn * j & 15))), to + 4 * j * kD);
+      LoadToLds(rows, 2 * (row * kD + 8 * (piece ^ (turn * j & 15))), to + 4 * j * kD);
     }
   };
   const auto load_k = [&](int64_t kb) { load(kbase, kb, (lane & 15) ^ lrow, 4, ks); };      // piece ^ row % 16
