@@ -1438,7 +1438,7 @@ void GpuMatMulQuantSwiGLU(const GpuTensor& w_gate, const GpuTensor& w_up, const 
     CheckGroup(mats, 2, outs);
     LaunchMatMulSmallSwiGLU(
         SmallOf(w_gate.type, static_cast<const uint8_t*>(w_gate.buf.data()), w_gate.rows, gate_dev),
-        SmallOf(w_up.type, static_cast<const uint8_t*>(w_up.buf.data()), w_up.rows, nullptr),
+        SmallOf(w_up.type, static_cast<const uint8_t*>(w_up.buf.data()), w_up.rows, up_dev),
         static_cast<int32_t>(w_gate.cols / kQK_K), x_dev, n_tokens);
     return;
   }

@@ -603,12 +603,13 @@ __global__ __launch_bounds__(64 * kW, kW == 8 ? 2 : kW == 10 ? 3 : 4) void MatMu
         gate = v;
       } else if (mine) {
         a.out[0][at] = dev::SiluMul(gate, v);
+        a.out[1][at] = v;
       }
     }
   }
 }
 
-// The sum of the K slices, in order. kSwiGLU: out[0] = silu(matrix 0) * matrix 1.
+// The sum of the K slices, in order. kSwiGLU: out[0] = silu(matrix 0) * matrix 1, out[1] = matrix 1.
 template <bool kSwiGLU>
 __global__ __launch_bounds__(256) void SmallReduceKernel(SmallArgs a, int32_t slices) {
   const int64_t per_mat = static_cast<int64_t>(a.n_tokens) * a.rows[0];
@@ -623,6 +624,7 @@ __global__ __launch_bounds__(256) void SmallReduceKernel(SmallArgs a, int32_t sl
     float u = p[0];
     for (int z = 1; z < slices; ++z) u += p[z * a.slice_elems];
     a.out[0][e] = dev::SiluMul(v, u);
+    a.out[1][e] = u;
   } else {
     int64_t at = e;
     int mi = 0;

@@ -26,7 +26,7 @@ void LaunchMatMulSmall(const SmallMat* mats, int32_t n_mats, int32_t nb, const f
 // the prefill GEMM (matmul_mfma.h). A rule on the matrix's own size.
 bool MatMulSmallWins(const SmallMat& m, int32_t nb, int64_t n_tokens);
 
-// gate.out <- silu(x . W_gate^T) * (x . W_up^T) for two matrices of one type and
+// up.out <- x . W_up^T, gate.out <- silu(x . W_gate^T) * up.out for two matrices of one type and
 // shape: the bits of LaunchMatMulSmall followed by GpuSiluMulInPlace.
 void LaunchMatMulSmallSwiGLU(const SmallMat& gate, const SmallMat& up, int32_t nb, const float* x, int64_t n_tokens);
 

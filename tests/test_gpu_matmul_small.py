@@ -80,6 +80,7 @@ def test_small_group_and_swiglu_equal_separate_calls(gpu, cols, n):
     gpu.GpuMatMulQuantSwiGLU(ws[3], ws[4], x, n, gate, up)
     gpu.GpuSiluMulInPlace(alone[3], alone[4], n * 9728)
     assert torch.equal(gate, alone[3])
+    assert torch.equal(up, alone[4]), "up holds its own product after a call of several tokens"
 
 
 @pytest.mark.parametrize("t", [Q4, Q6])
