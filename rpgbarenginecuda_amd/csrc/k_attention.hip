@@ -829,10 +829,13 @@ __global__ __launch_bounds__(kFused ? 64 * kFusedWaves : kBlockThreads) void Att
 // ---------------------------------------------------------------- prefill on the matrix cores
 //
 // Flash attention with v_mfma_f32_32x32x16_f16. One workgroup = one query head
-// and 128 consecutive tokens, 4 waves of 32 tokens; keys in blocks of 64 staged
-// in LDS as [key][dim] rows (16-byte writes) and shared by the waves; the V^T
-// fragments of the P.V step come out of the V rows through the transposing
-// LDS read (ds_read_b64_tr_b16).
+// and 128 consecutive tokens, 4 waves of 32 tokens; keys in blocks of 64 loaded
+// straight to LDS as [key][dim] rows, the next block while one is used, and shared
+// by the waves; the V^T fragments of the P.V step come out of the V rows through the
+// transposing LDS read (ds_read_b64_tr_b16). The products bound it (two for one, so
+// 57 us of 2811 tokens x 16 heads at a large product's rate), with the softmax beside
+// them: 92.6 us with each step's operands read from LDS as they were needed, 87.5 with
+// them read a step ahead.
 // Per wave and block:
 //   S^T (64 keys x 32 queries) = K . Q^T    2 key tiles x 8 dim steps x 2 terms
 //   O^T (128 dims x 32 queries) += V^T . P^T  4 dim tiles x 4 key steps x 2 terms
@@ -1415,7 +1418,7 @@ __global__ __launch_bounds__(256, 2) void AttnPrefillMfmaKernel(
 // sources are chosen so), which spreads both operands' reads over the banks. What
 // bounds it is the serial chain of a wave's blocks. 45 tokens at position 1500 (16 / 8
 // heads): 39 us with a wave per (token, kv head, key chunk), which reads the cache 45
-// times, 24 here.
+// times, 25 here.
 constexpr int kTurnRows = 32;
 constexpr int kTurnKeys = 32;
 constexpr int kTurnWaves = 8;
