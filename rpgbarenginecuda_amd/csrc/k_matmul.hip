@@ -1160,7 +1160,7 @@ bool SmallEligible(uint32_t type, const uint8_t* w_dev, const float* x_dev, int6
                    int64_t n_tokens) {
   return (type == kGgmlQ4_K || type == kGgmlQ6_K) && n_tokens >= 2 && n_tokens <= kSmallMaxTokens &&
          Aligned(x_dev, 16) && cols % kQK_K == 0 && Aligned(w_dev, type == kGgmlQ4_K ? 16 : 2) && rows <= INT32_MAX - 16 &&
-         cols <= INT32_MAX &&
+         cols < (int64_t{1} << 30) / n_tokens &&  // x has 32-bit byte offsets
          MatMulSmallWins(SmallOf(type, w_dev, rows, nullptr), static_cast<int32_t>(cols / kQK_K), n_tokens);
 }
 

@@ -38,6 +38,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cfloat>
 #include <type_traits>
 
 #include "dev_util.h"
@@ -121,6 +122,16 @@ __device__ __forceinline__ void LoadX(XRaw& x, const float* __restrict__ p) {
   }
 }
 
+// The same through a buffer, at (the lane's) + base (the wave's) bytes: one register for
+// the addresses instead of two.
+__device__ __forceinline__ void LoadX(XRaw& x, __amdgpu_buffer_rsrc_t rows, uint32_t at, uint32_t base) {
+#pragma unroll
+  for (int s = 0; s < kSteps; ++s)
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      x.v[s][k] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rows, static_cast<int>(at), static_cast<int>(base + 128 * s + 16 * k), 0));
+}
+
 // The value of the lane whose index differs in bit 0 / bit 1.
 __device__ __forceinline__ float Xor1(float v) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));
@@ -138,8 +149,8 @@ struct XSplit {
   double sum;
 };
 
-// inv: the wave's LDS area for the tokens' inverse scales.
-__device__ __forceinline__ void SplitX(const XRaw& x, XSplit& o, float* inv, int lane, bool want_sums) {
+// inv: the wave's LDS area for the tokens' inverse scales. Whether a value is infinite.
+__device__ __forceinline__ bool SplitX(const XRaw& x, XSplit& o, float* inv, int lane, bool want_sums) {
   float mx = 0.0f;
 #pragma unroll
   for (int s = 0; s < kSteps; ++s)
@@ -174,7 +185,8 @@ __device__ __forceinline__ void SplitX(const XRaw& x, XSplit& o, float* inv, int
     o.hi[s] = __builtin_bit_cast(F16x8, hm);
     o.lo[s] = __builtin_bit_cast(F16x8, lm);
   }
-  if (!want_sums) return;
+  const bool infinite = __builtin_amdgcn_ballot_w64(mx > FLT_MAX) != 0;
+  if (!want_sums) return infinite;
   // sums over a token's four lanes, transposed on the way: after two exchanges lane
   // 4 r + k holds the sum of step k
   const bool up2 = (lane & 2) != 0, up1 = (lane & 1) != 0;
@@ -186,6 +198,7 @@ __device__ __forceinline__ void SplitX(const XRaw& x, XSplit& o, float* inv, int
   // the token of lane r here)
   const int from_sum = 4 * (4 * (4 * (lane & 3) + ((lane >> 2) & 3)) + (lane >> 4));
   o.sum = __int_as_float(__builtin_amdgcn_ds_bpermute(from_sum, __float_as_int(total)));
+  return infinite;
 }
 
 // ---------------------------------------------------------------- weights
@@ -355,7 +368,35 @@ __device__ __forceinline__ void TileQ6(const WRaw<true>& w, const XSplit (&x)[kN
     for (int i = 0; i < 4; ++i) acc[nt][i] += (d * inv[nt][i]) * (hi[nt][i] + lo[nt][i]);
 }
 
+// ---------------------------------------------------------------- values that are not finite
+
+// Row `row` of a matrix times token t, each weight dequantised and added with one fused
+// multiply-add: what the tiled kernel of the smallest calls gives for infinities and NaNs.
+__device__ __forceinline__ float RowDot(bool q6, const uint8_t* w, int64_t row, int32_t nb, const float* x, int64_t t, int lane) {
+  const uint32_t type = q6 ? kGgmlQ6_K : kGgmlQ4_K;
+  const int32_t bytes = q6 ? kQ6KBlockBytes : kQ4KBlockBytes;
+  const uint8_t* wr = w + row * nb * bytes;
+  const float* xr = x + t * nb * kQK_K;
+  float acc = 0.0f;
+  for (int32_t b = 0; b < nb; ++b)
+#pragma unroll 1
+    for (int e = lane; e < kQK_K; e += 64)
+      acc = __builtin_fmaf(dev::DeqElemAny(type, wr + static_cast<int64_t>(b) * bytes, e), xr[static_cast<int64_t>(b) * kQK_K + e], acc);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+  return acc;
+}
+
 // ---------------------------------------------------------------- kernel
+
+// From this many tokens on a call stands for one of the prefill GEMM: the slices of a K
+// that is too long for a workgroup's registers become workgroups of their own, whose
+// partial results a second launch sums, and a token with a value that is not finite
+// gives NaNs. Below, a call stands for one of the tiled kernel: a workgroup walks the
+// slices itself, which needs no buffer (such calls never had one, so they may overlap on
+// several streams and be captured without a first run), and the results for infinities
+// are the tiled kernel's.
+constexpr int64_t kSliceMinTokens = 32;
 
 struct SmallArgs {
   const uint8_t* w[kSmallMaxMats];
@@ -409,11 +450,23 @@ __global__ __launch_bounds__(64 * kW, kW == 8 ? 2 : kW == 10 ? 3 : 4) void MatMu
   using C = SmallCfg<kW, kU, kNT, kAnyQ4, kAnyQ6, kSwiGLU>;
   constexpr int kToks = C::kToks;
   __shared__ __attribute__((aligned(16))) uint8_t lds[C::kBytes];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
+  __shared__ uint32_t lds_infinite[kW];
+  int tid = threadIdx.x;
+  int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int r = lane & 15;
-  const int kg = lane >> 4;
+  int r = lane & 15;
+  int kg = lane >> 4;
+  // The lane counted again, so that what follows from it isn't kept in registers until
+  // then: kLoop's 16 waves have 128 each, and a spilled address read back waits for all
+  // of the weights on their way.
+  auto lane_again = [&] {
+    uint32_t all = ~0u;
+    asm volatile("" : "+s"(all));
+    lane = static_cast<int>(__builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0u)));
+    tid = 64 * wave + lane;
+    r = lane & 15;
+    kg = lane >> 4;
+  };
   const int t0 = static_cast<int>(blockIdx.y) * kToks;
   const int n_here = a.n_tokens - t0 < kToks ? a.n_tokens - t0 : kToks;
   auto first_block = [&](int z) { return (static_cast<int>(blockIdx.z) + z) * a.bps; };
@@ -488,8 +541,10 @@ __global__ __launch_bounds__(64 * kW, kW == 8 ? 2 : kW == 10 ? 3 : 4) void MatMu
   Step now{0, 0}, next = after(now);
   // the slice's activations of this wave; past the slice: loaded, never used
   XRaw xr[kU][kNT];
+  const int64_t cols = static_cast<int64_t>(a.nb) * kQK_K;
+  // kLoop: n_tokens cols floats are less than 2^32 bytes
+  const __amdgpu_buffer_rsrc_t xrows = dev::OutResource(const_cast<float*>(a.x), 4u * static_cast<uint32_t>(a.n_tokens * cols));
   auto load_x = [&](int z) {
-    const int64_t cols = static_cast<int64_t>(a.nb) * kQK_K;
     const int units = 2 * blocks_of(z);
 #pragma unroll
     for (int k = 0; k < kU; ++k)
@@ -497,9 +552,17 @@ __global__ __launch_bounds__(64 * kW, kW == 8 ? 2 : kW == 10 ? 3 : 4) void MatMu
       for (int nt = 0; nt < kNT; ++nt) {
         const int u = kU * wave + k < units ? kU * wave + k : units - 1;
         const int t = t0 + 16 * nt + (lane >> 2);
-        LoadX(xr[k][nt], a.x + (t < a.n_tokens ? t : a.n_tokens - 1) * cols + kQK_K * first_block(z) + kUnit * u + 8 * (lane & 3));
+        const int64_t lane_at = (t < a.n_tokens ? t : a.n_tokens - 1) * cols + 8 * (lane & 3);
+        const int64_t wave_at = static_cast<int64_t>(kQK_K) * first_block(z) + kUnit * u;
+        if constexpr (kLoop) {
+          LoadX(xr[k][nt], xrows, 4u * static_cast<uint32_t>(lane_at), 4u * static_cast<uint32_t>(wave_at));
+        } else {
+          LoadX(xr[k][nt], a.x + (lane_at + wave_at));
+        }
       }
   };
+  bool infinite = false;  // among this wave's activations so far
+  if (lane == 0) lds_infinite[wave] = 0;
   // waves that have a unit of slice z; the others copy and sum
   auto waves_of = [&](int z) { return (2 * blocks_of(z) + kU - 1) / kU; };
   auto split_x = [&](int z) {
@@ -507,7 +570,8 @@ __global__ __launch_bounds__(64 * kW, kW == 8 ? 2 : kW == 10 ? 3 : 4) void MatMu
 #pragma unroll
     for (int k = 0; k < kU; ++k)
 #pragma unroll
-      for (int nt = 0; nt < kNT; ++nt) SplitX(xr[k][nt], xs[k][nt], invs + kToks * k + 16 * nt, lane, kAnyQ4);
+      for (int nt = 0; nt < kNT; ++nt) infinite |= SplitX(xr[k][nt], xs[k][nt], invs + kToks * k + 16 * nt, lane, kAnyQ4);
+    if (infinite) lds_infinite[wave] = 1;
   };
   load_x(0);
   load(now);
@@ -516,12 +580,14 @@ __global__ __launch_bounds__(64 * kW, kW == 8 ? 2 : kW == 10 ? 3 : 4) void MatMu
   stage(0);
   load(next);
   __syncthreads();
+  uint32_t flag = lds_infinite[lane % kW];  // (kLoop: of the first slice)
   for (int i = 0;; ++i, now = next, next = after(next)) {
     const int tile = tile_at(now.k);
     if (tile >= a.tiles) break;
     const int z = now.z;
     const int waves = waves_of(z);
     if constexpr (kLoop) {
+      if constexpr (kAnyQ6) lane_again();
       if (i > 0) {
         split_x(z);
         load_x(next.z);
@@ -607,6 +673,35 @@ __global__ __launch_bounds__(64 * kW, kW == 8 ? 2 : kW == 10 ? 3 : 4) void MatMu
       }
     }
   }
+  // An infinity's second term and 0 times it are NaNs that the sum of the weights' own
+  // products does not have: the outputs that are not finite again, each by its wave
+  if (a.n_tokens >= kSliceMinTokens) return;
+  lane_again();
+  if (kLoop) flag = lds_infinite[lane % kW];
+  if (__builtin_amdgcn_ballot_w64(flag != 0) == 0) return;
+  const int t = tid / (16 * C::kSum), c = (tid / C::kSum) & 15, part = tid % C::kSum;
+  for (int k = 0; tile_at(k) < a.tiles; k += kSwiGLU ? 2 : 1) {
+    int mi, r0;
+    locate(tile_at(k), &mi, &r0);
+    const bool mine = t < n_here && part == 0 && r0 + c < a.rows[mi];
+    const int64_t at = static_cast<int64_t>(t0 + t) * a.rows[mi] + r0 + c;
+    bool wrong = mine && !(fabsf(a.out[mi][at]) <= FLT_MAX);
+    if (kSwiGLU) wrong = wrong || (mine && !(fabsf(a.out[1][at]) <= FLT_MAX));
+    for (uint64_t left = __builtin_amdgcn_ballot_w64(wrong); left != 0; left &= left - 1) {
+      const int from = __builtin_ctzll(left);
+      const int row = r0 + __builtin_amdgcn_readlane(c, from), token = t0 + __builtin_amdgcn_readlane(t, from);
+      const float v = RowDot(is_q6(mi), a.w[mi], row, a.nb, a.x, token, lane);
+      if constexpr (kSwiGLU) {
+        const float u = RowDot(is_q6(1), a.w[1], row, a.nb, a.x, token, lane);
+        if (lane == from) {
+          a.out[0][at] = dev::SiluMul(v, u);
+          a.out[1][at] = u;
+        }
+      } else {
+        if (lane == from) a.out[mi][at] = v;
+      }
+    }
+  }
 }
 
 // The sum of the K slices, in order. kSwiGLU: out[0] = silu(matrix 0) * matrix 1, out[1] = matrix 1.
@@ -669,12 +764,6 @@ constexpr int kShapeCount = sizeof(kShapes) / sizeof(kShapes[0]);
 
 // How a launch of one workgroup shape covers a call: K slices of bps blocks,
 // groups of token tiles, row tiles per workgroup.
-//
-// The slices of a K that is too long for a workgroup's registers become workgroups
-// of their own, whose partial results a second launch sums; below kSliceMinTokens a
-// workgroup walks them itself, which needs no buffer (such calls never had one, so
-// they may overlap on several streams and be captured without a first run).
-constexpr int64_t kSliceMinTokens = 32;
 struct Plan {
   int bps, slices, loops, groups, grid, iters;
 };

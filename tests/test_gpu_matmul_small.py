@@ -121,3 +121,42 @@ def test_small_matmul_captures_without_a_first_run(gpu):
         gpu.GpuMatMulQuant(w, x, n, eager)
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
+
+
+@pytest.mark.parametrize("t,rows,cols,n", [(Q4, 6144, 2048, 21), (Q6, 6144, 2048, 12), (Q6, 2048, 6144, 21),
+                                           (Q4, 4000, 2560, 21)])
+def test_small_infinite_activation(gpu, ora, t, rows, cols, n):
+    """Below 32 tokens an infinite or NaN activation gives what the sum of the dequantised
+    weights' products gives (an infinity of the weight's sign, NaN where the weight is 0),
+    as the tiled kernel does; the other tokens keep their bits. Alone, in a group and
+    under SwiGLU."""
+    import torch
+
+    rng = np.random.default_rng(t + rows + cols + n)
+    raw = [synth.quant_table(rng, t, rows, cols) for _ in range(2)]
+    ws = [gpu.GpuTensor(dev(w), t, rows, cols) for w in raw]
+    x = rng.normal(0, 1, (n, cols)).astype(np.float32)
+    plain = torch.empty((n, rows), device="cuda")
+    gpu.GpuMatMulQuant(ws[0], dev(x), n, plain)
+    bad = [0, n // 2, n - 1]
+    x[bad[0], cols // 3] = -np.inf
+    x[bad[1], cols - 1] = np.inf
+    x[bad[2], 0] = np.nan
+    xd = dev(x)
+    outs = [torch.empty((n, rows), device="cuda") for _ in range(3)]
+    gpu.GpuMatMulQuant(ws[0], xd, n, outs[0])
+    gpu.GpuMatMulQuantGroup(ws, xd, n, outs[1:])
+    gate, up = torch.empty((n, rows), device="cuda"), torch.empty((n, rows), device="cuda")
+    gpu.GpuMatMulQuantSwiGLU(ws[0], ws[1], xd, n, gate, up)
+    wants = []
+    for w in raw:
+        w = ora.dequantize_row(t, w, rows * cols).reshape(rows, cols).astype(np.float64)
+        with np.errstate(invalid="ignore"):
+            wants.append(np.stack([(w * x[b].astype(np.float64)).sum(1) for b in bad]))
+    assert np.isinf(wants[0][:2]).any() and not np.isfinite(wants[0]).any()
+    good = [i for i in range(n) if i not in bad]
+    for out, want in ((outs[0], wants[0]), (outs[1], wants[0]), (outs[2], wants[1]), (up, wants[1])):
+        assert np.array_equal(host(out)[bad].astype(np.float64), want, equal_nan=True)
+    assert np.array_equal(host(outs[0])[good], host(plain)[good])
+    gpu.GpuSiluMulInPlace(outs[1], outs[2], n * rows)
+    assert np.array_equal(host(gate), host(outs[1]), equal_nan=True)
