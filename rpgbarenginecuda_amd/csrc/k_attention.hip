@@ -1445,7 +1445,10 @@ __global__ __launch_bounds__(64 * kTurnWaves, 1) void AttnTurnKernel(
   const bool qvalid = tq < seq;
   const int64_t pos0 = ReadPos0(pos0_val, pos0_dev);
   const bool full = t_first + kTurnRows <= seq;
-  const int64_t last_key = pos0 + (full ? t_first + kTurnRows : seq) - 1;  // the tile's causal limit
+  // The last keys that the tile's first token, this lane's and the tile's last one see. (The
+  // cache's end comes first only in a replayed graph with a bad staged pos0.)
+  const auto sees = [&](int64_t t) { return pos0 + t < max_seq ? pos0 + t : max_seq - 1; };
+  const int64_t first_key = sees(t_first), my_key = sees(tq), last_key = sees((full ? t_first + kTurnRows : seq) - 1);
 
   // a block's rows: load j takes rows 4 j + lane / 16, to piece lane % 16 (rows past
   // the causal limit repeat the last visible one: p = 0 meets finite values)
@@ -1503,8 +1506,8 @@ __global__ __launch_bounds__(64 * kTurnWaves, 1) void AttnTurnKernel(
     } else {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
-    const bool partly = kb + kTurnKeys - 1 > pos0 + t_first;  // some token does not see the whole block
-    const int64_t seen = qvalid ? pos0 + tq - kb : -1;        // offsets the lane's token sees, at most
+    const bool partly = kb + kTurnKeys - 1 > first_key;  // some token does not see the whole block
+    const int64_t seen = qvalid ? my_key - kb : -1;      // offsets the lane's token sees, at most
     // 0 times a value that is not finite would reach the tokens before it: such
     // values count as 0 in the products and are added for the tokens that see them
     uint64_t broken = 0;

@@ -114,3 +114,36 @@ def test_prefill_unaligned_values(gpu, seq):
     for v, out in ((dev(vc), outs[0]), (moved[2:2 + vc.size], outs[1])):
         gpu.GpuAttentionFromCache(nh, nkv, 128, pos0, dev(q), seq, dev(kc), v, max_seq, out)
     assert torch.equal(*outs)
+
+
+def test_turn_staged_past_the_cache(gpu, ora):
+    """A replay whose staged position puts tokens past the cache's end: they see the whole
+    cache, and nothing behind it is read (as the decode kernel does)."""
+    import torch
+
+    nh, nkv, max_seq, seq = 16, 8, 2048, 45
+    rng = np.random.default_rng(12)
+    q, kc, vc = make(rng, nh, nkv, max_seq, seq, qscale=0.5)
+    qd, kd, vd = dev(q), dev(kc), dev(vc)
+    out = torch.empty((seq, nh, 128), dtype=torch.float32, device="cuda")
+    gpu.init()
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        with gpu.ScopedEngineStream(stream):
+            graph.capture_begin()
+            gpu.GpuAttentionFromCache(nh, nkv, 128, 0, qd, seq, kd, vd, max_seq, out, max_seq)
+            graph.capture_end()
+    torch.cuda.synchronize()
+    for pos in (max_seq - 20, max_seq + 7):
+        gpu.stage_pos0(pos)
+        torch.cuda.synchronize()
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        got = host(out)
+        for t in (0, 19, 20, 33, 44):
+            at = min(pos + t, max_seq - 1)
+            ref, smag, vmax = ora.attention_f64(q[t:t + 1], kc, vc, max_seq, nh, nkv, 128, at, 1)
+            check(got[t:t + 1], ref, smag, vmax, at)
