@@ -1789,6 +1789,9 @@ void PlanGroupChunks(int64_t units, int64_t positions, int32_t* n_chunks, int64_
 // kMaxGroupChunks chunks): what a captured decode graph may replay.
 size_t WarmupFloats(int64_t /*positions*/) { return static_cast<size_t>(64) * kMaxGroupChunks * kPartFloats; }
 
+// Cache rows whose bytes the grouped decode kernel's offsets reach.
+constexpr int64_t kDecodeMaxSeq = INT32_MAX / (2 * kD);
+
 // A split grouped decode is one launch (AttnDecodeGroupKernel<G, kPrep, true>,
 // merged by the last workgroup of each pair), whatever the position budget: a
 // captured decode graph plans for the whole cache and replays at every position.
@@ -1800,7 +1803,7 @@ void LaunchDecodeGroup(const ModelMeta& c, const Pos0Arg& p0, const float* q_dev
   int32_t n_chunks;
   int64_t chunk_len;
   // the kernel forms (token, kv head) indices and chunk offsets in 32 bits
-  RPG_CHECK(seq * c.n_kv_heads < (int64_t{1} << 32) && max_seq <= INT32_MAX / (2 * kD),
+  RPG_CHECK(seq * c.n_kv_heads < (int64_t{1} << 32) && max_seq <= kDecodeMaxSeq,
             "decode attention over %lld (token, kv head) pairs and %lld cache rows exceeds the kernel's 32-bit "
             "indexing", static_cast<long long>(seq * c.n_kv_heads), static_cast<long long>(max_seq));
   PlanGroupChunks(seq * c.n_kv_heads, positions, &n_chunks, &chunk_len);
@@ -1857,12 +1860,14 @@ double DecodeUs(const ModelMeta& c, int64_t seq, int64_t positions) {
 // the groups measured; from 1024 positions on, where its error is no larger than the
 // decode kernel's: 2.0e-7 and 2.3e-7 for 45 tokens at 1500), with the alignment of the
 // 16-byte loads and stores. A call whose split decode the fixed region is too small
-// for stays with it, and is refused.
-bool TurnWins(const ModelMeta& c, const float* q_dev, int64_t seq, const uint16_t* v_layer, const float* out_dev,
-              int64_t positions, const PartialsSink& sink) {
+// for, or with a cache of more rows than the decode kernel indexes, stays with it, and is
+// refused.
+bool TurnWins(const ModelMeta& c, const float* q_dev, int64_t seq, const uint16_t* v_layer, int64_t max_seq,
+              const float* out_dev, int64_t positions, const PartialsSink& sink) {
   const int group = c.n_heads / c.n_kv_heads;
   const int64_t groups = (seq + kTurnRows - 1) / kTurnRows * c.n_heads;
-  if (seq < 2 || seq >= kFaMinTokens || positions < 1024 || (group != 1 && group != 2 && group != 4) || groups > 256 ||
+  if (seq < 2 || seq >= kFaMinTokens || positions < 1024 || max_seq > kDecodeMaxSeq ||
+      (group != 1 && group != 2 && group != 4) || groups > 256 ||
       ((reinterpret_cast<uintptr_t>(q_dev) | reinterpret_cast<uintptr_t>(v_layer) |
         reinterpret_cast<uintptr_t>(out_dev)) & 15u) != 0) {
     return false;
@@ -1906,7 +1911,7 @@ void AttentionFromCache(const ModelMeta& c, int64_t pos0, const float* q_dev, in
   int64_t chunk_len;
   PlanChunks(pairs, positions, &n_chunks, &chunk_len);
   const Pos0Arg p0 = Pos0ForLaunch(pos0);
-  if (TurnWins(c, q_dev, seq, v_layer, out_dev, positions, sink)) {
+  if (TurnWins(c, q_dev, seq, v_layer, max_seq, out_dev, positions, sink)) {
     LaunchTurn(c, p0, q_dev, seq, k_layer, v_layer, max_seq, scale, out_dev);
     return;
   }

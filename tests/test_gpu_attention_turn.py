@@ -147,3 +147,15 @@ def test_turn_staged_past_the_cache(gpu, ora):
             at = min(pos + t, max_seq - 1)
             ref, smag, vmax = ora.attention_f64(q[t:t + 1], kc, vc, max_seq, nh, nkv, 128, at, 1)
             check(got[t:t + 1], ref, smag, vmax, at)
+
+
+def test_turn_refuses_what_the_decode_kernel_refuses(gpu):
+    """A cache of more rows than the decode kernel's 32-bit indexing reaches is refused on the
+    host for a turn too (nothing is launched, so the buffers may be small)."""
+    import torch
+
+    nh, nkv, seq = 16, 4, 45
+    q = torch.zeros((seq, nh, 128), device="cuda")
+    kv = torch.zeros(4096, dtype=torch.int16, device="cuda")
+    with pytest.raises(gpu.RpgError, match="32-bit"):
+        gpu.GpuAttentionFromCache(nh, nkv, 128, 3000, q, seq, kv.data_ptr(), kv.data_ptr(), (2 ** 31 - 1) // 256 + 1, torch.empty_like(q))
