@@ -34,6 +34,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 #include <mutex>
 #include <utility>
@@ -1423,6 +1424,45 @@ constexpr int kTurnRows = 32;
 constexpr int kTurnKeys = 32;
 constexpr int kTurnWaves = 8;
 
+// One query row's output as the decode kernel forms it, products and sums in fp32: the dim
+// of lane % 16, whose column of the values v points to, over keys 0 .. last.
+__device__ __forceinline__ float TurnRowDim(const float* __restrict__ q, const uint16_t* __restrict__ k,
+                                            const uint16_t* __restrict__ v, int64_t last, float scale, int lane) {
+  float m = -INFINITY, l = 0.0f, o = 0.0f;
+#pragma unroll 1
+  for (int64_t kb = 0; kb <= last; kb += 64) {
+    const bool valid = kb + lane <= last;
+    const uint16_t* kr = k + (valid ? kb + lane : last) * kD;
+    float s = 0.0f;
+#pragma unroll 1
+    for (int i = 0; i < kD; i += 8) {
+      const uint4 w = *reinterpret_cast<const uint4*>(kr + i);
+      const uint32_t wd[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        s = __builtin_fmaf(q[i + 2 * j], HalfToF(wd[j] & 0xFFFFu), s);
+        s = __builtin_fmaf(q[i + 2 * j + 1], HalfToF(wd[j] >> 16), s);
+      }
+    }
+    s = valid ? s * scale : -INFINITY;
+    const float mn = fmaxf(m, WaveMax(s));
+    const float corr = mn == -INFINITY ? 1.0f : expf(m - mn);
+    const float p = valid ? expf(s - mn) : 0.0f;
+    l = l * corr + WaveSumF(p);
+    m = mn;
+    if (kb > 0) o *= corr;
+#pragma unroll 1
+    for (int i = 0; i < 16; ++i) {  // a quarter of the block's keys in each 16 lanes
+      const int j = 16 * (lane >> 4) + i;
+      const float pj = __shfl(p, j, 64);
+      if (kb + j <= last) o = __builtin_fmaf(pj, HalfToF(v[(kb + j) * kD]), o);
+    }
+  }
+  o += __shfl_xor(o, 16, 64);
+  o += __shfl_xor(o, 32, 64);
+  return o * (l > 0.0f ? 1.0f / l : 0.0f);
+}
+
 __global__ __launch_bounds__(64 * kTurnWaves, 1) void AttnTurnKernel(
     const float* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc, int64_t max_seq,
     int32_t n_heads, int32_t group, float scale, int64_t pos0_val, const int64_t* __restrict__ pos0_dev, int64_t seq,
@@ -1568,10 +1608,10 @@ __global__ __launch_bounds__(64 * kTurnWaves, 1) void AttnTurnKernel(
       sums(wv)[(8 * dt + 2 * g + hf) * kTurnRows + col] =
           make_float4(o[dt][4 * g] * f, o[dt][4 * g + 1] * f, o[dt][4 * g + 2] * f, o[dt][4 * g + 3] * f);
   __syncthreads();
-  if (!qvalid) return;
   // wave wv finishes dims 16 wv .. + 15: 4 of them, 8 g + 4 hf .. + 3, in each lane
   const float inv = L > 0.0f ? 1.0f / L : 0.0f;
   float* orow = out + (tq * n_heads + h) * kD + 16 * wv + 4 * hf;
+  uint32_t broken = 0;  // bit 4 g + i: dim 8 g + 4 hf + i is not finite
 #pragma unroll
   for (int g = 0; g < 2; ++g) {
     float4 acc = sums(0)[(4 * wv + 2 * g + hf) * kTurnRows + col];
@@ -1580,7 +1620,26 @@ __global__ __launch_bounds__(64 * kTurnWaves, 1) void AttnTurnKernel(
       const float4 v = sums(w)[(4 * wv + 2 * g + hf) * kTurnRows + col];
       acc = make_float4(acc.x + v.x, acc.y + v.y, acc.z + v.z, acc.w + v.w);
     }
-    *reinterpret_cast<float4*>(orow + 8 * g) = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+    acc = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+    if (qvalid) {
+      *reinterpret_cast<float4*>(orow + 8 * g) = acc;
+      const float e[4] = {acc.x, acc.y, acc.z, acc.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) broken |= (fabsf(e[i]) <= FLT_MAX ? 0u : 1u) << (4 * g + i);
+    }
+  }
+  const uint64_t lanes = __builtin_amdgcn_ballot_w64(broken != 0);
+  if (lanes == 0) return;
+  // An infinity's product with the second term of a probability or a query is a NaN that
+  // the product with their sum may not be: what is not finite again, in fp32
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // behind the stores above
+  for (uint32_t rows = static_cast<uint32_t>(lanes | lanes >> 32); rows != 0; rows &= rows - 1) {
+    const int row = __builtin_ctz(rows);
+    const int dim = lane & 15;
+    const int64_t th = (t_first + row) * n_heads + h;
+    const float v = TurnRowDim(q + th * kD, kbase, vbase + 16 * wv + dim, sees(t_first + row), scale, lane);
+    const bool bad = ((__shfl(broken, row + 8 * (dim & 4), 64) >> ((dim >> 1 & 4) + (dim & 3))) & 1u) != 0;
+    if (lane < 16 && bad) out[th * kD + 16 * wv + dim] = v;
   }
 }
 

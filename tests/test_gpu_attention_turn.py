@@ -159,3 +159,63 @@ def test_turn_refuses_what_the_decode_kernel_refuses(gpu):
     kv = torch.zeros(4096, dtype=torch.int16, device="cuda")
     with pytest.raises(gpu.RpgError, match="32-bit"):
         gpu.GpuAttentionFromCache(nh, nkv, 128, 3000, q, seq, kv.data_ptr(), kv.data_ptr(), (2 ** 31 - 1) // 256 + 1, torch.empty_like(q))
+
+
+def reference(q, kc, vc, max_seq, nkv, pos0):
+    """Causal attention in float64 with its infinities: [seq, heads, 128]."""
+    seq, nh = q.shape[:2]
+    k = kc.reshape(nkv, max_seq, 128).view(np.float16).astype(np.float64)
+    v = vc.reshape(nkv, max_seq, 128).view(np.float16).astype(np.float64)
+    out = np.empty((seq, nh, 128))
+    with np.errstate(invalid="ignore"):
+        for t in range(seq):
+            n = pos0 + t + 1
+            for h in range(nh):
+                j = h // (nh // nkv)
+                s = (k[j, :n] * q[t, h].astype(np.float64)).sum(1) / np.sqrt(128)
+                p = np.exp(s - s.max())
+                out[t, h] = (p[:, None] * v[j, :n]).sum(0) / p.sum()
+    return out
+
+
+@pytest.mark.parametrize("key", [0, 100, 1499, 1500, 1503])
+def test_turn_infinities_in_the_history(gpu, key):
+    """An infinite value of a token that the whole tile sees is that infinity in its dim (and
+    other dims and kv heads keep their bits); an infinite key leaves its token out where the
+    score is -inf and gives NaN where it is +inf. As the decode kernel does."""
+    import torch
+
+    nh, nkv, max_seq, pos0, seq = 16, 8, 2048, 1500, 45
+    rng = np.random.default_rng(key)
+    q, kc, vc = make(rng, nh, nkv, max_seq, seq, qscale=0.5)
+    q[:, :, 5] = np.abs(q[:, :, 5]) + np.float32(0.1)
+
+    def run(k, v):
+        out = torch.empty((seq, nh, 128), dtype=torch.float32, device="cuda")
+        args = (nh, nkv, 128, pos0, dev(q), seq, dev(k.reshape(-1)), dev(v.reshape(-1)), max_seq, out)
+        assert takes_it(gpu, lambda: gpu.GpuAttentionFromCache(*args))
+        return host(out)
+
+    plain = run(kc, vc)
+    first = max(key - pos0, 0)  # the first token that sees it
+    v = vc.copy().reshape(nkv, max_seq, 128)
+    v[3, key, 77] = np.float16(-np.inf).view(np.uint16)
+    got = run(kc, v)
+    assert np.all(got[first:, 6:8, 77] == -np.inf)
+    rest = np.ones(plain.shape, bool)
+    rest[first:, 6:8, 77] = False
+    assert np.array_equal(got[rest], plain[rest])
+    v[3, key - 1 if key else 1, 77] = np.float16(np.inf).view(np.uint16)
+    assert np.all(np.isnan(run(kc, v)[max(key - pos0, 1):, 6:8, 77]))
+
+    k = kc.copy().reshape(nkv, max_seq, 128)
+    k[3, key, 5] = np.float16(-np.inf).view(np.uint16)
+    got = run(k, vc)
+    rest = np.ones(plain.shape, bool)
+    rest[first:, 6:8] = False
+    assert np.array_equal(got[rest], plain[rest])
+    # scores and values of size 1: 1e-5 is 80 roundings of 2^-23
+    assert np.allclose(got, reference(q, k, vc, max_seq, nkv, pos0), rtol=0, atol=1e-5)
+    k[3, key, 5] = np.float16(np.inf).view(np.uint16)
+    got = run(k, vc)
+    assert np.all(np.isnan(got[first:, 6:8])) and np.array_equal(got[rest], plain[rest])
