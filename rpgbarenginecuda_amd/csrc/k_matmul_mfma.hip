@@ -31,7 +31,6 @@
 // workgroups share a CU and cover each other's barriers and LDS latency.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <cmath>
 #include <mutex>
 
@@ -1261,25 +1260,19 @@ int64_t PlanesSlice(bool q4, int32_t nb) {
   return slice < tile ? tile : slice;
 }
 
-// A whole matrix on the planes: its time (per slice, the decode's launch and its bytes,
-// the GEMM's launch and plan), and the buffers that it takes.
-struct PlanesNeed {
+// A whole matrix on the planes, in us: per slice, the decode's launch and its bytes, the
+// GEMM's launch and plan.
+double PlanesMatrixUs(bool q4, int64_t rows, int32_t nb, int64_t n_tokens) {
+  const int64_t tile = q4 ? PlanesCfg<kGgmlQ4_K>::kTileR : PlanesCfg<kGgmlQ6_K>::kTileR;
+  const int64_t slice = PlanesSlice(q4, nb);
   double us = 0.0;
-  size_t weights = 0, partials = 0;
-  PlanesNeed(bool q4, int64_t rows, int32_t nb, int64_t n_tokens) {
-    const int64_t tile = q4 ? PlanesCfg<kGgmlQ4_K>::kTileR : PlanesCfg<kGgmlQ6_K>::kTileR;
-    const int64_t slice = PlanesSlice(q4, nb);
-    for (int64_t r = 0; r < rows; r += slice) {
-      const int64_t n = rows - r < slice ? rows - r : slice;
-      const int64_t tiles = (n_tokens + kTileT - 1) / kTileT * ((n + tile - 1) / tile);
-      const PlanesLayout lay(q4, n, nb);
-      const PlanesPlan plan = PlanFor(q4, tiles, nb);
-      us += 4.5 + static_cast<double>(lay.bytes) / 4e6 + 4.0 + plan.us;
-      weights = std::max(weights, lay.bytes);
-      partials = std::max(partials, static_cast<size_t>(tiles - plan.dp) * plan.splits * kTileT * tile * sizeof(float));
-    }
+  for (int64_t r = 0; r < rows; r += slice) {
+    const int64_t n = rows - r < slice ? rows - r : slice;
+    const int64_t tiles = (n_tokens + kTileT - 1) / kTileT * ((n + tile - 1) / tile);
+    us += 4.5 + static_cast<double>(PlanesLayout(q4, n, nb).bytes) / 4e6 + 4.0 + PlanFor(q4, tiles, nb).us;
   }
-};
+  return us;
+}
 
 template <uint32_t kType>
 void LaunchPlanesRows(const uint8_t* w, int64_t rows, int64_t row_bytes, int32_t nb, const SplitActivations& sa,
@@ -1331,11 +1324,6 @@ void LaunchPlanes(const uint8_t* w, int64_t rows, int64_t row_bytes, int32_t nb,
   }
 }
 
-bool Holds(SplitBuffer& b, size_t bytes) {
-  std::lock_guard<std::mutex> lock(b.mu);
-  return b.bytes >= bytes;
-}
-
 }  // namespace
 
 // From four token tiles on: 9728 x 2560 Q4_K at 448 tokens 92 us on the planes and 105 on
@@ -1343,7 +1331,7 @@ bool Holds(SplitBuffer& b, size_t bytes) {
 // is too much of it (72 and 76 us at 333 tokens from caches, but 4% slower with weights
 // that come from memory).
 double PlanesUs(bool q6, int64_t rows, int32_t nb, int64_t n_tokens) {
-  return n_tokens < kPlanesFewTokens ? HUGE_VAL : PlanesNeed(!q6, rows, nb, n_tokens).us;
+  return n_tokens < kPlanesFewTokens ? HUGE_VAL : PlanesMatrixUs(!q6, rows, nb, n_tokens);
 }
 
 // The GEMM that decodes per 128-token tile: 20 us, more for a long K, and about 280
@@ -1397,10 +1385,6 @@ void LaunchMatMulMfmaSplit(uint32_t type, const uint8_t* w, int64_t rows, int64_
   if (on_planes && sa.n_tokens < kPlanesMinTokens) {
     on_planes = sa.n_tokens >= kPlanesFewTokens &&
                 PlanesUs(type == kGgmlQ6_K, rows, nb, sa.n_tokens) < MfmaUs(rows, nb, sa.n_tokens);
-    if (on_planes && StreamIsCapturing()) {  // nothing may be allocated: only if the shape ran before
-      const PlanesNeed need(type == kGgmlQ4_K, rows, nb, sa.n_tokens);
-      on_planes = Holds(WeightPlanes(), need.weights) && Holds(PartialTiles(), need.partials);
-    }
   }
   if (on_planes) {
     if (type == kGgmlQ4_K) {

@@ -4,6 +4,10 @@ token tiles, one block to several, against the float64 oracle within the bound o
 tests/test_gpu_matmul.py."""
 from __future__ import annotations
 
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -30,3 +34,72 @@ def test_planes_matmul_vs_f64(gpu, ora, t, rows, cols, n):
     exact, absdot = ora.matmul_quant_f64(t, w, rows, cols, x)
     check(host(out[:n]), exact, absdot, cols, factored_magnitude(ora, t, w, rows, cols, x))
     assert torch.isnan(out[n]).all(), "wrote past the last token"
+
+
+CAPTURE = """
+import torch
+from rpgbarenginecuda_amd import ops
+
+ops.init()
+gen = torch.Generator(device="cuda")
+gen.manual_seed(1)
+
+
+def matrix(t, rows):
+    nb, bb = rows * 10, ops.BLOCK_BYTES[t]
+    b = torch.randint(0, 256, (nb, bb), generator=gen, device="cuda", dtype=torch.uint8)
+    b[:, slice(0, 4) if t == 12 else slice(208, 210)] = 20  # the fp16 scales: 0x1414
+    return ops.GpuTensor(b.reshape(-1), t, rows, 2560)
+
+
+def capture(w, x, out, refused):
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    stream.wait_stream(torch.cuda.current_stream())
+    with ops.ScopedEngineStream(stream), torch.cuda.stream(stream):
+        graph.capture_begin()
+        try:
+            ops.GpuMatMulQuant(w, x, len(x), out)
+            assert not refused, "captured without its buffers"
+        except ops.RpgError as e:
+            assert refused and "run the same shape once before capturing" in str(e), e
+        finally:
+            graph.capture_end()
+    torch.cuda.synchronize()
+    return graph
+
+
+def kernels(call):
+    ops.profile_start(16)
+    call()
+    ops.profile_stop()
+    return set(ops.profile_report())
+
+
+w, other = matrix(12, 9728), matrix(14, 9728)
+x = torch.randn(448, 2560, generator=gen, device="cuda")
+out, eager = (torch.empty(448, 9728, device="cuda") for _ in range(2))
+# the activations' buffer, from a call on the GEMM that decodes as it goes
+assert "MatMulMfmaQ6KKernel" in kernels(lambda: ops.GpuMatMulQuant(other, x[:385], 385, eager))
+assert "MatMulMfmaQ6KKernel" in kernels(lambda: ops.GpuMatMulQuant(other, x, 448, eager))
+capture(w, x, out, True)
+assert "MatMulMfmaQ4KPlanesKernel" in kernels(lambda: ops.GpuMatMulQuant(w, x, 448, eager))
+graph = capture(w, x, out, False)
+for scale in (1.0, -2.0, 0.5):
+    x *= scale
+    out.fill_(float("nan"))
+    graph.replay()
+    ops.GpuMatMulQuant(w, x, 448, eager)
+    torch.cuda.synchronize()
+    assert torch.equal(out, eager)
+print("done", flush=True)
+"""
+
+
+def test_planes_capture_takes_the_eager_route():
+    """448 tokens on a matrix that runs on the planes, in a process of its own (the library's
+    buffers only grow): captured before the shape has run, with the activations' buffer
+    there from another call, it is refused and not sent to another kernel; after a run,
+    replays give the eager bits."""
+    repo = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    run = subprocess.run([sys.executable, "-c", CAPTURE], cwd=repo, timeout=100, capture_output=True, text=True)
+    assert run.returncode == 0 and "done" in run.stdout, run.stderr[-2000:]
