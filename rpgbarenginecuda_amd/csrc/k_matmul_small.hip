@@ -819,7 +819,7 @@ void LaunchTyped(const char* name, SmallArgs a, int32_t n_mats, bool any4, bool 
   }
   if (p.slices > 1) {
     const int64_t n = kSwiGLU ? static_cast<int64_t>(a.n_tokens) * a.rows[0] : a.slice_elems;
-    Launch("MatMulSplitReduceKernel", SmallReduceKernel<kSwiGLU>, dim3(GridFor(n, 256)), dim3(256), a,
+    Launch("MatMulSmallReduceKernel", SmallReduceKernel<kSwiGLU>, dim3(GridFor(n, 256)), dim3(256), a,
            static_cast<int32_t>(p.slices));
   }
 }
@@ -844,11 +844,10 @@ void LaunchShaped(int shape, const SmallMat* mats, int32_t n_mats, int32_t nb, c
     }
     a.tile_end[i] = i + 1 < n_mats ? a.tiles : INT32_MAX;
   }
-  const bool prompt = n_tokens >= 32;
-  const char* name = kSwiGLU        ? (any6 ? "MatMulSwiGLUQ6KKernel" : "MatMulSwiGLUQ4KKernel")
-                     : any4 && any6 ? (prompt ? "MatMulMfmaQ4KQ6KSmallKernel" : "MatMulQ4KQ6KKernel")
-                     : any6         ? (prompt ? "MatMulMfmaQ6KSmallKernel" : "MatMulQ6KKernel")
-                                    : (prompt ? "MatMulMfmaQ4KSmallKernel" : "MatMulQ4KKernel");
+  const char* name = kSwiGLU        ? (any6 ? "MatMulSmallSwiGLUQ6KKernel" : "MatMulSmallSwiGLUQ4KKernel")
+                     : any4 && any6 ? "MatMulSmallQ4KQ6KKernel"
+                     : any6         ? "MatMulSmallQ6KKernel"
+                                    : "MatMulSmallQ4KKernel";
   switch (shape) {
     case 0:
       if (PlanFor(0, nb, n_tokens, a.tiles).loops > 1) return LaunchTyped<0, kSwiGLU, true>(name, a, n_mats, any4, any6);

@@ -1,8 +1,8 @@
 """Path equivalence of the quantised matmul (GpuSetForceGenericMatMul,
 src/kernels_gpu.h:51-58; the reference's bitwise generic-vs-specialised check,
 tools/matmul_bench.cu:149-219): every specialised kernel -- the one-token decode
-matvecs (2 and 4 rows per wave, and the split-columns form), the tiled
-small-batch kernel and the matrix-core prefill GEMM with and without split K,
+matvecs (2 and 4 rows per wave, and the split-columns form), the tiled kernel, the
+small-batch matrix-core kernel and the prefill GEMM with and without split K,
 decoding per tile or from decoded weight planes --
 against the generic per-element kernel on the same weights and inputs.
 
@@ -49,8 +49,7 @@ def exact_table(rng, qtype, rows, cols):
 
 
 CASES = [
-    # (name, type, rows, cols, n_tokens, specialised kernel the call must take: a name prefix, the
-    # matrix-core kernels having a ping-pong form for small grids)
+    # (name, type, rows, cols, n_tokens, the launches that the call must take)
     ("decode Q4_K, 2 rows per wave", Q4_K, 2048, 2048, 1, "MatVecQ4KKernel"),
     ("decode Q4_K, 4 rows per wave", Q4_K, 32768, 2048, 1, "MatVecQ4KKernel"),
     ("decode Q6_K", Q6_K, 1024, 2048, 1, "MatVecQ6KKernel"),
@@ -58,19 +57,37 @@ CASES = [
     ("decode Q6_K, tall matrix", Q6_K, 16400, 2048, 1, "MatVecQ6KKernel"),
     ("decode Q6_K, tall, 10 blocks per row", Q6_K, 16384, 2560, 1, "MatVecSplitQ6KKernel"),
     ("decode Q4_K, split columns", Q4_K, 1024, 4096, 1, "MatVecSplitQ4KKernel"),
-    ("small batch Q4_K", Q4_K, 2048, 2048, 8, "MatMulQ4KKernel"),
-    ("small batch Q6_K", Q6_K, 1024, 2048, 5, "MatMulQ6KKernel"),
-    ("matrix cores Q4_K", Q4_K, 6144, 2048, 300, "MatMulMfmaQ4K"),
-    ("matrix cores Q6_K", Q6_K, 2048, 6144, 300, "MatMulMfmaQ6K"),
-    ("matrix cores Q4_K, split K", Q4_K, 1024, 2048, 48, "MatMulSplitReduceKernel"),
-    ("decoded weight planes Q4_K", Q4_K, 6144, 2048, 700, "MatMulMfmaQ4KPlanes"),
-    ("decoded weight planes Q6_K", Q6_K, 2048, 2048, 600, "MatMulMfmaQ6KPlanes"),
-    ("decoded weight planes Q4_K, split K, ragged", Q4_K, 1152, 2048, 513, "MatMulMfmaQ4KPlanes"),
-    ("decoded weight planes Q4_K, whole rounds + split tail", Q4_K, 4352, 512, 2048, "MatMulPlanesReduceKernel"),
-    ("decoded weight planes Q6_K, whole rounds + split tail", Q6_K, 2176, 512, 2000, "MatMulPlanesReduceKernel"),
+    ("tiled Q4_K", Q4_K, 1024, 2048, 5, "MatMulQ4KKernel"),
+    ("tiled Q6_K", Q6_K, 1024, 2048, 5, "MatMulQ6KKernel"),
+    ("small batch Q4_K", Q4_K, 2048, 2048, 8, "MatMulSmallQ4KKernel"),
+    ("small batch Q6_K, K slices in one workgroup", Q6_K, 2048, 6144, 21, "MatMulSmallQ6KKernel"),
+    ("small batch Q4_K, medium prompt", Q4_K, 6144, 2048, 300, "MatMulSmallQ4KKernel"),
+    ("small batch Q6_K, medium prompt, K slices summed", Q6_K, 2048, 6144, 300,
+     "MatMulSmallQ6KKernel MatMulSmallReduceKernel"),
+    ("small batch Q4_K, short prompt", Q4_K, 1024, 2048, 48, "MatMulSmallQ4KKernel MatMulSmallReduceKernel"),
+    ("matrix cores Q4_K, split K", Q4_K, 9728, 2560, 333,
+     "SplitActivationsKernel MatMulMfmaQ4KKernel MatMulSplitReduceKernel"),
+    ("matrix cores Q6_K", Q6_K, 9728, 2560, 400, "SplitActivationsKernel MatMulMfmaQ6KKernel"),
+    ("matrix cores Q6_K, split K, ragged", Q6_K, 4100, 2560, 300,
+     "SplitActivationsKernel MatMulMfmaQ6KKernel MatMulSplitReduceKernel"),
+    ("matrix cores Q6_K, two chunks at a time, split K", Q6_K, 9728, 2560, 128,
+     "SplitActivationsKernel MatMulMfmaQ6KPingPongKernel MatMulSplitReduceKernel"),
+    ("matrix cores Q4_K, two chunks at a time, split K", Q4_K, 13808, 4352, 110,
+     "SplitActivationsKernel MatMulMfmaQ4KPingPongKernel MatMulSplitReduceKernel"),
+    ("decoded weight planes Q4_K", Q4_K, 6144, 2048, 700, "PrepareQ4KKernel MatMulMfmaQ4KPlanesKernel"),
+    ("decoded weight planes Q6_K", Q6_K, 2048, 2048, 600,
+     "PrepareQ6KKernel MatMulMfmaQ6KPlanesKernel MatMulPlanesReduceKernel"),
+    ("decoded weight planes Q4_K, split K, ragged", Q4_K, 1152, 2048, 513,
+     "PrepareQ4KKernel MatMulMfmaQ4KPlanesKernel MatMulPlanesReduceKernel"),
+    ("decoded weight planes Q4_K, whole rounds + split tail", Q4_K, 4352, 512, 2048,
+     "PrepareQ4KKernel MatMulMfmaQ4KPlanesKernel MatMulPlanesReduceKernel"),
+    ("decoded weight planes Q6_K, whole rounds + split tail", Q6_K, 2176, 512, 2000,
+     "PrepareQ6KKernel MatMulMfmaQ6KPlanesKernel MatMulPlanesReduceKernel"),
     ("decoded weight planes Q6_K above 64 MB: two row slices, the last ragged", Q6_K, 8300, 2048, 512,
-     "MatMulMfmaQ6KPlanes"),
-    ("decoded weight planes Q4_K, 10 blocks per row (4B shape)", Q4_K, 1024, 2560, 520, "MatMulMfmaQ4KPlanes"),
+     "PrepareQ6KKernel DecodeWeightPlanesQ6KKernel MatMulMfmaQ6KPlanesKernel MatMulPlanesReduceKernel"),
+    ("decoded weight planes Q4_K, 10 blocks per row (4B shape)", Q4_K, 1024, 2560, 520,
+     "PrepareQ4KKernel MatMulMfmaQ4KPlanesKernel MatMulPlanesReduceKernel"),
+    ("decoded weight planes Q4_K below 512 tokens", Q4_K, 9728, 2560, 448, "PrepareQ4KKernel MatMulMfmaQ4KPlanesKernel"),
 ]
 
 
@@ -94,8 +111,8 @@ def _run(gpu, qtype, w, rows, cols, x, n_tokens, force_generic):
     return out.cpu().numpy(), kernels
 
 
-@pytest.mark.parametrize("name,qtype,rows,cols,n_tokens,kernel", CASES, ids=[c[0] for c in CASES])
-def test_specialised_equals_generic_bit_for_bit(gpu, ora, name, qtype, rows, cols, n_tokens, kernel):
+@pytest.mark.parametrize("name,qtype,rows,cols,n_tokens,kernels", CASES, ids=[c[0] for c in CASES])
+def test_specialised_equals_generic_bit_for_bit(gpu, ora, name, qtype, rows, cols, n_tokens, kernels):
     import torch
 
     _case(f"generic vs specialised: {name} [{rows} x {cols}] x {n_tokens} tokens")
@@ -109,7 +126,7 @@ def test_specialised_equals_generic_bit_for_bit(gpu, ora, name, qtype, rows, col
     xd = torch.from_numpy(x).cuda()
     spec, k_spec = _run(gpu, qtype, w, rows, cols, xd, n_tokens, False)
     gen, k_gen = _run(gpu, qtype, w, rows, cols, xd, n_tokens, True)
-    assert any(k.startswith(kernel) for k in k_spec), k_spec
+    assert k_spec == set(kernels.split())
     assert k_gen == {"MatMulGenericKernel"}, k_gen
     assert not gpu.GpuForceGenericMatMul()
     assert np.array_equal(spec.view(np.uint32), gen.view(np.uint32)), \
