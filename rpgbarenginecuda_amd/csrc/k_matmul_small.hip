@@ -899,10 +899,6 @@ void LaunchMatMulSmall(const SmallMat* mats, int32_t n_mats, int32_t nb, const f
     }
     double us = 0.0;
     shape_of_all = ShapeOf(rows, any6, nb, n_tokens, &us);
-    // 33 to 64 tokens of at most 1024 rows: in K slices whatever the cost says (8.9
-    // against 7.1 us at 1024 x 2048 x 64 tokens, 22.3 on the prefill GEMM), so that the
-    // sliced form of a short K stays in use where the GEMM's had been.
-    if (n_tokens > 32 && n_tokens <= 64 && rows <= 1024) shape_of_all = 2;
   }
   for (int shape = 0; shape < kShapeCount; ++shape) {
     SmallMat same[kSmallMaxMats];

@@ -64,7 +64,7 @@ CASES = [
     ("small batch Q4_K, medium prompt", Q4_K, 6144, 2048, 300, "MatMulSmallQ4KKernel"),
     ("small batch Q6_K, medium prompt, K slices summed", Q6_K, 2048, 6144, 300,
      "MatMulSmallQ6KKernel MatMulSmallReduceKernel"),
-    ("small batch Q4_K, short prompt", Q4_K, 1024, 2048, 48, "MatMulSmallQ4KKernel MatMulSmallReduceKernel"),
+    ("small batch Q4_K, short prompt", Q4_K, 1024, 2048, 48, "MatMulSmallQ4KKernel"),
     ("matrix cores Q4_K, split K", Q4_K, 9728, 2560, 333,
      "SplitActivationsKernel MatMulMfmaQ4KKernel MatMulSplitReduceKernel"),
     ("matrix cores Q6_K", Q6_K, 9728, 2560, 400, "SplitActivationsKernel MatMulMfmaQ6KKernel"),

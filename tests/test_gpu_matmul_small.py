@@ -13,6 +13,13 @@ pytestmark = pytest.mark.gpu
 
 Q4, Q6 = 12, 14
 
+def launches(gpu, call):
+    gpu.profile_start(16)
+    call()
+    gpu.profile_stop()
+    return set(gpu.profile_report())
+
+
 SHAPES = [
     # (type, rows, cols, tokens)
     (Q4, 1, 256, 5), (Q6, 1, 256, 6),            # one row, one block
@@ -160,3 +167,17 @@ def test_small_infinite_activation(gpu, ora, t, rows, cols, n):
     assert np.array_equal(host(outs[0])[good], host(plain)[good])
     gpu.GpuSiluMulInPlace(outs[1], outs[2], n * rows)
     assert np.array_equal(host(gate), host(outs[1]), equal_nan=True)
+
+
+@pytest.mark.parametrize("n", [33, 48, 64])
+def test_small_short_prompt_of_a_shard_is_one_launch(gpu, n):
+    """q / k / v of a tensor-parallel shard (512 rows of 2048 columns): K fits the workgroups, so
+    there are no slices to sum."""
+    import torch
+
+    rng = np.random.default_rng(n)
+    ws = [gpu.GpuTensor(dev(synth.quant_table(rng, t, r, 2048)), t, r, 2048) for t, r in ((Q4, 256), (Q4, 128), (Q6, 128))]
+    x = dev(rng.normal(0, 1, (n, 2048)).astype(np.float32))
+    outs = [torch.empty((n, w.rows), device="cuda") for w in ws]
+    assert launches(gpu, lambda: gpu.GpuMatMulQuantGroup(ws, x, n, outs)) == {"MatMulSmallQ4KQ6KKernel"}
+    assert launches(gpu, lambda: gpu.GpuMatMulQuant(ws[0], x, n, outs[0])) == {"MatMulSmallQ4KKernel"}
