@@ -1420,15 +1420,13 @@ void LaunchMatMulMfmaSplit(uint32_t type, const uint8_t* w, int64_t rows, int64_
            pp ? MatMulMfmaKernel<kGgmlQ6_K, true> : MatMulMfmaKernel<kGgmlQ6_K, false>, grid, block, w, rows,
            row_bytes, nb, planes, sums, sa.sum_stride, sa.inv_scale, sa.cols, sa.n_tokens, bps, out, partial);
   }
-  if (splits > 1) LaunchSplitReduce(partial, elems, splits, out);
+  if (splits > 1) {
+    Launch("MatMulSplitReduceKernel", MatMulSplitReduceKernel, dim3(GridFor(elems, kThreads)), dim3(kThreads),
+           static_cast<const float*>(partial), elems, splits, out);
+  }
 }
 
 float* SplitPartials(size_t bytes) { return static_cast<float*>(EnsurePartialTiles(bytes)); }
-
-void LaunchSplitReduce(const float* partial, int64_t elems, int32_t splits, float* out) {
-  Launch("MatMulSplitReduceKernel", MatMulSplitReduceKernel, dim3(GridFor(elems, kThreads)), dim3(kThreads), partial,
-         elems, splits, out);
-}
 
 void LaunchMatMulMfma(uint32_t type, const uint8_t* w, int64_t rows, int64_t row_bytes, int32_t nb, const float* x,
                       int64_t cols, int64_t n_tokens, float* out) {

@@ -5,10 +5,10 @@
 // the latency of one pass (load, decode, multiply, combine) and, as rows and tokens
 // add up, by the vector instructions that decode the weights. One launch does it all,
 // with nothing prepared beforehand:
-//   * a workgroup takes a K slice of up to 8 or 16 half blocks and walks tiles of 16
-//     weight rows; its waves split the slice, each keeping its half blocks of all the
-//     tokens in registers, so the activations are read and split once per workgroup
-//     and a weight is decoded once per 16 or 32 tokens;
+//   * a workgroup takes a K slice of up to 8 to 20 half blocks (by its shape) and walks
+//     tiles of 16 weight rows; its waves split the slice, each keeping its half blocks
+//     of all the tokens in registers, so the activations are read and split once per
+//     workgroup and a weight is decoded once per 16 or 32 tokens;
 //   * within a half block K runs in four steps of 32 columns, one Q4_K sub-block or
 //     Q6_K quarter each: lane (r, kg) = (lane % 16, lane / 16) holds columns 32 s +
 //     8 kg .. + 7 of token r (A of v_mfma_f32_16x16x32_f16) and of weight row r (B);
@@ -735,24 +735,15 @@ __global__ __launch_bounds__(256) void SmallReduceKernel(SmallArgs a, int32_t sl
   }
 }
 
-// Row tiles over the matrices (pairs of them for SwiGLU).
-template <bool kSwiGLU>
-void SetTiles(SmallArgs* a, int32_t n_mats) {
-  a->tiles = 0;
-  for (int i = 0; i < kSmallMaxMats; ++i) {
-    if (i < n_mats) a->tiles += (a->rows[i] + 15) / 16;
-    a->tile_end[i] = i + 1 < n_mats ? a->tiles : INT32_MAX;
-  }
-}
-
 // Workgroup shapes (waves, half blocks per wave, token tiles) and what they cost:
 // a fixed part (launch, activations, first and last tile) and a part per row tile
-// that a workgroup walks, by weight type. Measured on MI355X over n = 16 .. 448 at
-// the 1.7B and 4B layer matrices (graph replay): us = fixed + tiles * step fits each
-// within 10%, e.g. 2048 x 2048 Q4_K at 16 / 448 tokens 6.8 / 23.8 us, 2048 x 6144
-// Q6_K at 21 tokens 15.1 us. 16 waves and one token tile are quickest for few tokens
-// and few tiles; two token tiles share a decode and win as the tiles add up; 10
-// waves fit rows of 10 blocks in two slices.
+// that a workgroup walks, by weight type: us = fixed + tiles * step. Against MI355X
+// times (graph replay, weights from memory) at 214 sizes of 4 .. 448 tokens on the
+// 1.7B and 4B layer matrices it gives 0.81 to 1.22 of them, nine in ten between 0.84
+// and 1.13: 2048 x 2048 Q4_K at 21 / 448 tokens 7.0 / 24.0 us (measured 7.1 / 27.4),
+// 2048 x 6144 Q6_K at 21 tokens 14.4 (16.2). 16 waves and one token tile are quickest
+// for few tokens and few tiles; two token tiles share a decode and win as the tiles
+// add up; 10 waves fit rows of 10 blocks in two slices.
 struct Shape {
   int w, u, nt;
   double fixed, step4, step6;
@@ -773,8 +764,7 @@ Plan PlanFor(int shape, int nb, int64_t n_tokens, int want) {
   const int nt = s.nt, blocks = s.w * s.u / 2;
   Plan p;
   p.slices = (nb + blocks - 1) / blocks;
-  // up to 8 blocks: slices of 4, whose sums are those of the unsliced shapes' tree
-  p.bps = nb <= 8 && p.slices > 1 ? 4 : (nb + p.slices - 1) / p.slices;
+  p.bps = (nb + p.slices - 1) / p.slices;
   p.slices = (nb + p.bps - 1) / p.bps;
   p.loops = 1;
   if (n_tokens < kSliceMinTokens) {
@@ -859,12 +849,13 @@ void LaunchShaped(int shape, const SmallMat* mats, int32_t n_mats, int32_t nb, c
   }
 }
 
-// The shape for `rows` rows, and its cost. Up to 8 blocks the first three shapes sum in
-// one order, so a group may take the shape of its rows together; a longer row's
-// order depends on the shape, which then comes from the matrix's own rows.
+// The shape for `rows` rows, and its cost. Up to 8 blocks (4 for the third shape) the
+// first shapes hold whole rows and sum in one order, so a group may take the shape of
+// its rows together; a longer row's order depends on the shape, which then comes from
+// the matrix's own rows.
 int ShapeOf(int64_t rows, bool q6, int32_t nb, int64_t n_tokens, double* us) {
   int best = 0;
-  for (int i = 0; i < (nb <= 8 ? 3 : kShapeCount); ++i) {
+  for (int i = 0; i < (nb <= 4 ? 3 : nb <= 8 ? 2 : kShapeCount); ++i) {
     const double c = ShapeCost(i, nb, n_tokens, rows, q6);
     if (i == 0 || c < *us) {
       best = i;

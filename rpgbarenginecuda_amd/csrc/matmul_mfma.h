@@ -43,10 +43,8 @@ double PlanesUs(bool q6, int64_t rows, int32_t nb, int64_t n_tokens);
 double MfmaUs(int64_t rows, int32_t nb, int64_t n_tokens);
 
 // A library-owned buffer of at least `bytes` for the partial results of K slices
-// (valid until the next split launch on the engine stream), and the launch that
-// sums them: out[e] = sum over z < splits of partial[z elems + e], in that order.
+// (valid until the next split launch on the engine stream).
 float* SplitPartials(size_t bytes);
-void LaunchSplitReduce(const float* partial, int64_t elems, int32_t splits, float* out);
 
 }  // namespace rpg
 
