@@ -1368,6 +1368,7 @@ bool MakeNorm(const GpuNormIn& in, int64_t cols, NormPrologue* nrm) {
 void GpuMatMulQuantGroup(const GpuTensor* const* ws, int32_t n_mats, const float* x_dev, int64_t n_tokens,
                          float* const* outs) {
   CheckGroup(ws, n_mats, outs);
+  RPG_CHECK(x_dev != nullptr, "GpuMatMulQuantGroup got a null pointer");
   const int64_t cols = ws[0]->cols;
   if (g_force_generic.load()) {
     for (int32_t i = 0; i < n_mats; ++i) GpuMatMulQuant(*ws[i], x_dev, n_tokens, outs[i]);

@@ -181,3 +181,15 @@ def test_small_short_prompt_of_a_shard_is_one_launch(gpu, n):
     outs = [torch.empty((n, w.rows), device="cuda") for w in ws]
     assert launches(gpu, lambda: gpu.GpuMatMulQuantGroup(ws, x, n, outs)) == {"MatMulSmallQ4KQ6KKernel"}
     assert launches(gpu, lambda: gpu.GpuMatMulQuant(ws[0], x, n, outs[0])) == {"MatMulSmallQ4KKernel"}
+
+
+@pytest.mark.parametrize("n", [1, 8, 21, 64, 600])
+def test_group_refuses_null_activations(gpu, n):
+    """On the host, whatever kernel the group would take (nothing is launched)."""
+    import torch
+
+    rng = np.random.default_rng(n)
+    ws = [gpu.GpuTensor(dev(synth.quant_table(rng, t, 2048, 2048)), t, 2048, 2048) for t in (Q4, Q6)]
+    outs = [torch.empty((n, 2048), device="cuda") for _ in ws]
+    with pytest.raises(gpu.RpgError, match="null pointer"):
+        gpu.GpuMatMulQuantGroup(ws, None, n, outs)
