@@ -1152,21 +1152,17 @@ namespace {
 // The small-batch kernel takes Q4_K / Q6_K matrices under the same alignment
 // rules, up to kSmallMaxTokens tokens (from there on the decoded-planes GEMM) and
 // where it is the faster one.
-constexpr int64_t kSmallMaxTokens = 511;
+constexpr int64_t kSmallMinTokens = 2, kSmallMaxTokens = 511;
 SmallMat SmallOf(uint32_t type, const uint8_t* w_dev, int64_t rows, float* out) {
   return SmallMat{w_dev, out, rows, type == kGgmlQ6_K};
 }
 bool SmallEligible(uint32_t type, const uint8_t* w_dev, const float* x_dev, int64_t rows, int64_t cols,
                    int64_t n_tokens) {
-  return (type == kGgmlQ4_K || type == kGgmlQ6_K) && n_tokens >= 2 && n_tokens <= kSmallMaxTokens &&
+  return (type == kGgmlQ4_K || type == kGgmlQ6_K) && n_tokens >= kSmallMinTokens && n_tokens <= kSmallMaxTokens &&
          Aligned(x_dev, 16) && cols % kQK_K == 0 && Aligned(w_dev, type == kGgmlQ4_K ? 16 : 2) && rows <= INT32_MAX - 16 &&
          cols < (int64_t{1} << 30) / n_tokens &&  // x has 32-bit byte offsets
          MatMulSmallWins(SmallOf(type, w_dev, rows, nullptr), static_cast<int32_t>(cols / kQK_K), n_tokens);
 }
-
-}  // namespace
-
-namespace {
 
 // GpuSetForceGenericMatMul: while set, every matmul entry point runs
 // MatMulGenericKernel (per-element decode, one wave per output) so the
@@ -1376,24 +1372,26 @@ void GpuMatMulQuantGroup(const GpuTensor* const* ws, int32_t n_mats, const float
   }
   // A few tokens: the matrices share launches. The others of the group follow as
   // a group of their own.
-  std::vector<SmallMat> small;
   std::vector<const GpuTensor*> rest;
   std::vector<float*> rest_outs;
-  for (int32_t i = 0; i < n_mats; ++i) {
-    const uint8_t* w = static_cast<const uint8_t*>(ws[i]->buf.data());
-    if (SmallEligible(ws[i]->type, w, x_dev, ws[i]->rows, cols, n_tokens)) {
-      small.push_back(SmallOf(ws[i]->type, w, ws[i]->rows, outs[i]));
-    } else {
-      rest.push_back(ws[i]);
-      rest_outs.push_back(outs[i]);
+  if (n_tokens >= kSmallMinTokens && n_tokens <= kSmallMaxTokens) {
+    std::vector<SmallMat> small;
+    for (int32_t i = 0; i < n_mats; ++i) {
+      const uint8_t* w = static_cast<const uint8_t*>(ws[i]->buf.data());
+      if (SmallEligible(ws[i]->type, w, x_dev, ws[i]->rows, cols, n_tokens)) {
+        small.push_back(SmallOf(ws[i]->type, w, ws[i]->rows, outs[i]));
+      } else {
+        rest.push_back(ws[i]);
+        rest_outs.push_back(outs[i]);
+      }
     }
-  }
-  if (!small.empty()) {
-    LaunchMatMulSmall(small.data(), static_cast<int32_t>(small.size()), static_cast<int32_t>(cols / kQK_K), x_dev, n_tokens);
-    if (rest.empty()) return;
-    ws = rest.data();
-    outs = rest_outs.data();
-    n_mats = static_cast<int32_t>(rest.size());
+    if (!small.empty()) {
+      LaunchMatMulSmall(small.data(), static_cast<int32_t>(small.size()), static_cast<int32_t>(cols / kQK_K), x_dev, n_tokens);
+      if (rest.empty()) return;
+      ws = rest.data();
+      outs = rest_outs.data();
+      n_mats = static_cast<int32_t>(rest.size());
+    }
   }
   // Prefill: the activations are split once for all the matrices (each output
   // bit-identical to its own GpuMatMulQuant call, which splits the same way).
