@@ -933,7 +933,9 @@ __device__ __forceinline__ F16x8 SplitTerm(float (&x)[8]) {
 }
 
 // A query row as the matrix core's operand (B of the scores): lane (col, hf) holds
-// its own query's dims, the two terms of q 2^e scale log2(e); *sinv = 2^-e.
+// its own query's dims, the two terms of q 2^e scale log2(e); *sinv = 2^-e. kFine: the
+// second term is that of the exact product, so only the terms round.
+template <bool kFine>
 __device__ __forceinline__ void FaLoadQ(const float* __restrict__ qrow, bool qvalid, float scale, int hf,
                                         F16x8 (&qb)[2][8], float* sinv) {
   // ---- q row: this lane holds dims 16 s + 8 hf + j (s = 0..7), the partner lane the rest
@@ -965,17 +967,20 @@ __device__ __forceinline__ void FaLoadQ(const float* __restrict__ qrow, bool qva
   *sinv = ldexpf(1.0f, -e);
 #pragma unroll
   for (int s = 0; s < 8; ++s) {
+    float exact[8];  // the products' remainders
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      qv[s][j] *= qmul;
+      const float q = qv[s][j];
+      qv[s][j] = q * qmul;
       // the rounded product, and not the exact one: given the choice the compiler
       // rounds q qmul to fp16 in one step for one use and in two for another, and
       // where they differ the remainder belongs to another first term (a row in
       // 300 was off by 1e-4 relative)
       asm("" : "+v"(qv[s][j]));
+      exact[j] = __builtin_fmaf(q, qmul, -static_cast<float>(static_cast<_Float16>(qv[s][j])));
     }
     qb[0][s] = SplitTerm(qv[s]);
-    qb[1][s] = SplitTerm(qv[s]);
+    qb[1][s] = SplitTerm(kFine ? exact : qv[s]);
   }
 }
 
@@ -1182,7 +1187,7 @@ __global__ __launch_bounds__(256, 2) void AttnPrefillMfmaKernel(
 
   F16x8 qb[2][8];
   float sinv;
-  FaLoadQ(q + (tq * n_heads + h) * kD, qvalid, scale, hf, qb, &sinv);
+  FaLoadQ<false>(q + (tq * n_heads + h) * kD, qvalid, scale, hf, qb, &sinv);
 
   F32x16 o[4];
 #pragma unroll
@@ -1522,7 +1527,7 @@ __global__ __launch_bounds__(64 * kTurnWaves, 1) void AttnTurnKernel(
 
   F16x8 qb[2][8];
   float sinv;
-  FaLoadQ(q + ((qvalid ? tq : 0) * n_heads + h) * kD, qvalid, scale, hf, qb, &sinv);
+  FaLoadQ<true>(q + ((qvalid ? tq : 0) * n_heads + h) * kD, qvalid, scale, hf, qb, &sinv);
   F32x16 o[4];
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt) o[dt] = F32x16{};
@@ -1609,18 +1614,23 @@ __global__ __launch_bounds__(64 * kTurnWaves, 1) void AttnTurnKernel(
           make_float4(o[dt][4 * g] * f, o[dt][4 * g + 1] * f, o[dt][4 * g + 2] * f, o[dt][4 * g + 3] * f);
   __syncthreads();
   // wave wv finishes dims 16 wv .. + 15: 4 of them, 8 g + 4 hf .. + 3, in each lane
-  const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+  // (summed and scaled in double: what is left of the error is the products')
+  const double inv = L > 0.0f ? 1.0 / static_cast<double>(L) : 0.0;
   float* orow = out + (tq * n_heads + h) * kD + 16 * wv + 4 * hf;
   uint32_t broken = 0;  // bit 4 g + i: dim 8 g + 4 hf + i is not finite
 #pragma unroll
   for (int g = 0; g < 2; ++g) {
-    float4 acc = sums(0)[(4 * wv + 2 * g + hf) * kTurnRows + col];
+    double sum[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int w = 1; w < kTurnWaves; ++w) {
+    for (int w = 0; w < kTurnWaves; ++w) {
       const float4 v = sums(w)[(4 * wv + 2 * g + hf) * kTurnRows + col];
-      acc = make_float4(acc.x + v.x, acc.y + v.y, acc.z + v.z, acc.w + v.w);
+      sum[0] += v.x;
+      sum[1] += v.y;
+      sum[2] += v.z;
+      sum[3] += v.w;
     }
-    acc = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+    const float4 acc = make_float4(static_cast<float>(sum[0] * inv), static_cast<float>(sum[1] * inv),
+                                   static_cast<float>(sum[2] * inv), static_cast<float>(sum[3] * inv));
     if (qvalid) {
       *reinterpret_cast<float4*>(orow + 8 * g) = acc;
       const float e[4] = {acc.x, acc.y, acc.z, acc.w};
@@ -1916,8 +1926,9 @@ double DecodeUs(const ModelMeta& c, int64_t seq, int64_t positions) {
 
 // Calls for AttnTurnKernel: 2 to kFaMinTokens - 1 tokens where the decode kernel takes
 // longer than its 7 us and 2.35 us a block of every wave (with a tenth to spare, for
-// the groups measured; from 1024 positions on, where its error is no larger than the
-// decode kernel's: 2.0e-7 and 2.3e-7 for 45 tokens at 1500), with the alignment of the
+// the groups measured; from 1024 positions on, where its error is below the decode
+// kernel's: 1.9e-7 and 2.2e-7 for 45 tokens at 1500, 0.85 of it at the median of 42
+// sizes and 0.98 at most), with the alignment of the
 // 16-byte loads and stores. A call whose split decode the fixed region is too small
 // for, or with a cache of more rows than the decode kernel indexes, stays with it, and is
 // refused.

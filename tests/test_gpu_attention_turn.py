@@ -219,3 +219,20 @@ def test_turn_infinities_in_the_history(gpu, key):
     k[3, key, 5] = np.float16(np.inf).view(np.uint16)
     got = run(k, vc)
     assert np.all(np.isnan(got[first:, 6:8])) and np.array_equal(got[rest], plain[rest])
+
+
+@pytest.mark.parametrize("nh,nkv,pos0,seq,decode", [(32, 8, 1500, 21, 1.891e-7), (16, 4, 1024, 63, 1.891e-7),
+                                                       (16, 8, 1500, 45, 2.2e-7)])
+def test_turn_error_is_below_the_decode_kernels(gpu, ora, nh, nkv, pos0, seq, decode):
+    """Queries, probabilities and sums as two fp16 terms lose nothing against the fp32 kernel
+    that took these calls: `decode` is that kernel's error (2-norm, relative) on these inputs."""
+    import torch
+
+    max_seq = 2048
+    rng = np.random.default_rng(pos0 + seq)
+    q, kc, vc = make(rng, nh, nkv, max_seq, seq)
+    out = torch.empty((seq, nh, 128), dtype=torch.float32, device="cuda")
+    gpu.GpuAttentionFromCache(nh, nkv, 128, pos0, dev(q), seq, dev(kc), dev(vc), max_seq, out)
+    ref = ora.attention_f64(q, kc, vc, max_seq, nh, nkv, 128, pos0, seq)[0]
+    err = float(np.linalg.norm(host(out).astype(np.float64) - ref) / np.linalg.norm(ref))
+    assert err <= decode
