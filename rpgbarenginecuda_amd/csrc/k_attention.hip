@@ -1912,26 +1912,29 @@ void LaunchDecodeGroup(const ModelMeta& c, const Pos0Arg& p0, const float* q_dev
   }
 }
 
-// What the decode kernel takes for several tokens, in us: it reads the cache once per
-// (token, kv head), so n_kv tokens positions times a rate that grows with the heads of a
-// group, and more once the (token, kv head) pairs leave fewer key chunks each (measured:
-// 16 / 8 heads, 21 tokens at 1500 17 us, 31 at 3000 46, 45 at 1500 39; 32 / 8 heads, 21
-// at 3000 42, 45 at 1500 63).
-double DecodeUs(const ModelMeta& c, int64_t seq, int64_t positions) {
-  const int group = c.n_heads / c.n_kv_heads;
-  const double units = static_cast<double>(seq * c.n_kv_heads);
-  const double rate = (group <= 1 ? 3.5e-5 : group <= 2 ? 4.4e-5 : 7.2e-5) * (units >= 256 ? 1.35 : 1.0);
-  return 5.0 + units * static_cast<double>(positions) * rate;
+// What the two kernels take for a turn, in us (graph replay, 1210 sizes of 2 to 63 tokens
+// at 1024 to 4000 and 4 to 64 heads in groups of 1, 2 and 4, with keys and values from
+// memory). The decode kernel reads the cache once per (token, kv head): a rate that grows
+// with the heads of a group, and three quarters of it where the pairs' workgroups all run
+// at once, two on a CU (8 / 8 heads at 3000: 31 tokens 33 us, 32 tokens 24, 33 tokens
+// 32). The other one walks all of the keys in each workgroup, whatever the tokens
+// and heads: 17 us at 1024, 21 at 1500, 35 at 3000.
+double DecodeUs(int group, int64_t units, int64_t positions, int32_t n_chunks) {
+  const bool at_once = units <= 256 && n_chunks <= 2 * kFusedWaves;
+  const double rate = (group <= 1 ? 3.2e-5 : group <= 2 ? 4.8e-5 : 7.2e-5) * (at_once ? 0.75 : 1.0);
+  return 8.0 + static_cast<double>(units) * static_cast<double>(positions) * rate;
 }
+double TurnUs(int64_t positions) { return 6.85 + 9.3e-3 * static_cast<double>(positions); }
 
-// Calls for AttnTurnKernel: 2 to kFaMinTokens - 1 tokens where the decode kernel takes
-// longer than its 7 us and 2.35 us a block of every wave (with a tenth to spare, for
-// the groups measured; from 1024 positions on, where its error is below the decode
-// kernel's: 1.9e-7 and 2.2e-7 for 45 tokens at 1500, 0.85 of it at the median of 42
-// sizes and 0.98 at most), with the alignment of the
-// 16-byte loads and stores. A call whose split decode the fixed region is too small
-// for, or with a cache of more rows than the decode kernel indexes, stays with it, and is
-// refused.
+// Calls for AttnTurnKernel: 2 to kFaMinTokens - 1 tokens of the groups measured where that
+// is faster by 6% or more: of the sizes above, three then take up to 5% longer than on the
+// decode kernel (17.3 against 16.5 us), where blocks of 2.35 us and no regard for pairs
+// that run at once sent 31 to the slower one, up to 1.56 times (8 / 8 heads, 32 tokens at
+// 4000: 47 against 30 us). From 1024 positions on, where its error is below the decode
+// kernel's (1.9e-7 and 2.2e-7 for 45 tokens at 1500, 0.85 of it at the median of 42 sizes
+// and 0.98 at most), with the alignment of the 16-byte loads and stores. A call whose
+// split decode the fixed region is too small for, or with a cache of more rows than the
+// decode kernel indexes, stays with it, and is refused.
 bool TurnWins(const ModelMeta& c, const float* q_dev, int64_t seq, const uint16_t* v_layer, int64_t max_seq,
               const float* out_dev, int64_t positions, const PartialsSink& sink) {
   const int group = c.n_heads / c.n_kv_heads;
@@ -1947,8 +1950,7 @@ bool TurnWins(const ModelMeta& c, const float* q_dev, int64_t seq, const uint16_
   PlanGroupChunks(seq * c.n_kv_heads, positions, &n_chunks, &chunk_len);
   const int64_t n_groups = (n_chunks + kFusedWaves - 1) / kFusedWaves;
   if (n_groups > 1 && static_cast<size_t>(seq * c.n_heads * n_groups * kPartFloats) > sink.Capacity()) return false;
-  const int64_t blocks = (positions + kTurnKeys * kTurnWaves - 1) / (kTurnKeys * kTurnWaves);
-  return 1.1 * (7.0 + 2.35 * static_cast<double>(blocks)) < DecodeUs(c, seq, positions);
+  return 1.06 * TurnUs(positions) < DecodeUs(group, seq * c.n_kv_heads, positions, n_chunks);
 }
 
 void LaunchTurn(const ModelMeta& c, const Pos0Arg& p0, const float* q_dev, int64_t seq, const uint16_t* k_layer,

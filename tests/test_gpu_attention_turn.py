@@ -29,6 +29,24 @@ def takes_it(gpu, call):
     return set(gpu.profile_report()) == {"AttnTurnKernel"}
 
 
+# (n_heads, n_kv_heads, pos0, seq, whether the matrix-core kernel was measured to be the faster one)
+ROUTES = [
+    (8, 8, 3000, 32, False), (8, 8, 4000, 32, False), (16, 16, 2200, 16, False), (32, 32, 4000, 8, False),
+    (8, 8, 4000, 33, False), (16, 8, 3000, 32, False), (16, 8, 1500, 21, False),
+    (16, 8, 1500, 45, True), (32, 8, 1500, 21, True), (16, 4, 1500, 45, True), (8, 8, 1500, 40, True),
+    (16, 16, 3000, 31, True), (64, 16, 1500, 12, True),
+]
+
+
+@pytest.mark.parametrize("nh,nkv,pos0,seq,turn", ROUTES)
+def test_turn_route_is_the_faster_kernel(gpu, nh, nkv, pos0, seq, turn):
+    import torch
+
+    q = torch.zeros((seq, nh, 128), device="cuda")
+    kv = torch.zeros(nkv * 4200 * 128, dtype=torch.int16, device="cuda")
+    assert takes_it(gpu, lambda: gpu.GpuAttentionFromCache(nh, nkv, 128, pos0, q, seq, kv, kv, 4200, torch.empty_like(q))) == turn
+
+
 @pytest.mark.parametrize("nh,nkv,max_seq,pos0,seq", CASES)
 def test_turn_vs_f64(gpu, ora, nh, nkv, max_seq, pos0, seq):
     import torch
