@@ -1614,7 +1614,8 @@ __global__ __launch_bounds__(64 * kTurnWaves, 1) void AttnTurnKernel(
           make_float4(o[dt][4 * g] * f, o[dt][4 * g + 1] * f, o[dt][4 * g + 2] * f, o[dt][4 * g + 3] * f);
   __syncthreads();
   // wave wv finishes dims 16 wv .. + 15: 4 of them, 8 g + 4 hf .. + 3, in each lane
-  // (summed and scaled in double: what is left of the error is the products')
+  // (pairs of waves summed and scaled in double: with all of it in float up to 4% more error
+  // than the decode kernel's, with every wave in double half a microsecond more)
   const double inv = L > 0.0f ? 1.0 / static_cast<double>(L) : 0.0;
   float* orow = out + (tq * n_heads + h) * kD + 16 * wv + 4 * hf;
   uint32_t broken = 0;  // bit 4 g + i: dim 8 g + 4 hf + i is not finite
@@ -1622,12 +1623,13 @@ __global__ __launch_bounds__(64 * kTurnWaves, 1) void AttnTurnKernel(
   for (int g = 0; g < 2; ++g) {
     double sum[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int w = 0; w < kTurnWaves; ++w) {
-      const float4 v = sums(w)[(4 * wv + 2 * g + hf) * kTurnRows + col];
-      sum[0] += v.x;
-      sum[1] += v.y;
-      sum[2] += v.z;
-      sum[3] += v.w;
+    for (int w = 0; w < kTurnWaves / 2; ++w) {
+      const float4 u = sums(w)[(4 * wv + 2 * g + hf) * kTurnRows + col];
+      const float4 v = sums(w + kTurnWaves / 2)[(4 * wv + 2 * g + hf) * kTurnRows + col];
+      sum[0] += u.x + v.x;
+      sum[1] += u.y + v.y;
+      sum[2] += u.z + v.z;
+      sum[3] += u.w + v.w;
     }
     const float4 acc = make_float4(static_cast<float>(sum[0] * inv), static_cast<float>(sum[1] * inv),
                                    static_cast<float>(sum[2] * inv), static_cast<float>(sum[3] * inv));
@@ -1927,14 +1929,13 @@ double DecodeUs(int group, int64_t units, int64_t positions, int32_t n_chunks) {
 double TurnUs(int64_t positions) { return 6.85 + 9.3e-3 * static_cast<double>(positions); }
 
 // Calls for AttnTurnKernel: 2 to kFaMinTokens - 1 tokens of the groups measured where that
-// is faster by 6% or more: of the sizes above, three then take up to 5% longer than on the
-// decode kernel (17.3 against 16.5 us), where blocks of 2.35 us and no regard for pairs
-// that run at once sent 31 to the slower one, up to 1.56 times (8 / 8 heads, 32 tokens at
-// 4000: 47 against 30 us). From 1024 positions on, where its error is below the decode
-// kernel's (1.9e-7 and 2.2e-7 for 45 tokens at 1500, 0.85 of it at the median of 42 sizes
-// and 0.98 at most), with the alignment of the 16-byte loads and stores. A call whose
-// split decode the fixed region is too small for, or with a cache of more rows than the
-// decode kernel indexes, stays with it, and is refused.
+// is faster by 6% or more. (45 tokens at 1500: 22 us against 39 with 16 / 8 heads, 22 and
+// 37 with 16 / 4; 32 tokens at 4000 with 8 / 8 heads 47 and 30. Of the sizes above three
+// take up to 5% longer here than there.) From 1024 positions on, where its error is below
+// the decode kernel's (1.9e-7 and 2.2e-7 for 45 tokens at 1500, 0.89 of it at the median
+// of 42 sizes and no more at any), with the alignment of the 16-byte loads and stores. A
+// call whose split decode the fixed region is too small for, or with a cache of more rows
+// than the decode kernel indexes, stays with it, and is refused.
 bool TurnWins(const ModelMeta& c, const float* q_dev, int64_t seq, const uint16_t* v_layer, int64_t max_seq,
               const float* out_dev, int64_t positions, const PartialsSink& sink) {
   const int group = c.n_heads / c.n_kv_heads;
