@@ -1334,12 +1334,50 @@ double PlanesUs(bool q6, int64_t rows, int32_t nb, int64_t n_tokens) {
   return n_tokens < kPlanesFewTokens ? HUGE_VAL : PlanesMatrixUs(!q6, rows, nb, n_tokens);
 }
 
-// The GEMM that decodes per 128-token tile: 20 us, more for a long K, and about 280
-// useful TFLOP/s (1024 x 2048 Q4_K: 24.5 us at 128 tokens, 29 at 448; 2560 x 9728 Q6_K:
-// 75 and 149).
-double MfmaUs(int64_t rows, int32_t nb, int64_t n_tokens) {
-  const double mega = static_cast<double>(rows) * 256e-6 * nb;  // weights, in millions
-  return 20.0 + 0.02 * nb * nb + 2.0 * static_cast<double>((n_tokens + 127) / 128 * 128) * mega / 280.0;
+namespace {
+
+// How the GEMM that decodes per tile covers a matrix. When the output tiles cannot give
+// every CU a workgroup, K is divided into slices of whole blocks whose partial tiles are
+// summed afterwards in a fixed order (deterministic). Between one and two workgroups per
+// CU the extra pass costs more than the second workgroup slot gains.
+struct GemmPlan {
+  int64_t gx, gy, tiles;
+  int32_t bps, splits;
+  bool pp;
+};
+GemmPlan PlanGemm(int64_t rows, int32_t nb, int64_t n_tokens) {
+  constexpr int64_t kFill = 256;
+  GemmPlan p;
+  p.gx = (rows + kTileR - 1) / kTileR;
+  p.gy = (n_tokens + kTileT - 1) / kTileT;
+  p.tiles = p.gx * p.gy;
+  int64_t want = p.tiles >= kFill ? 1 : (kFill + p.tiles - 1) / p.tiles;
+  if (want > nb) want = nb;
+  p.bps = static_cast<int32_t>((nb + want - 1) / want);
+  p.splits = static_cast<int32_t>((nb + p.bps - 1) / p.bps);
+  // wide matrices (more than 16 row tiles) only while the token tiles are
+  // mostly empty: ffn_gate measured 14% faster at 130 tokens, 9% slower at 256
+  p.pp = p.tiles <= kPingPongTiles && (p.gx <= 16 || n_tokens <= 160);
+  return p;
+}
+
+}  // namespace
+
+// The split of the activations, a workgroup's blocks as often as its CU takes one, and
+// the reduce; two workgroups on a CU take a quarter longer than one. Of MI355X times at
+// 32 to 511 tokens and 129 to 32000 rows of 1 to 56 blocks nine in ten are met within
+// 15%: 9728 x 2560 Q4_K at 300 tokens 67 us (74 measured), Q6_K 98 (99).
+double MfmaUs(bool q6, int64_t rows, int32_t nb, int64_t n_tokens) {
+  const GemmPlan p = PlanGemm(rows, nb, n_tokens);
+  const int64_t groups = p.tiles * p.splits;
+  if (p.pp) {
+    const double n = static_cast<double>(n_tokens) * 1e-6;  // in millions
+    const double reduce = p.splits > 1 ? 1.5 + 2.24 * (p.splits + 1) * n * static_cast<double>(rows) : 0.0;
+    return 13.0 + static_cast<double>(p.bps * ((groups + 255) / 256)) * (q6 ? 5.9 : 4.0) + reduce + 6.6 * n * kQK_K * nb;
+  }
+  const int64_t rest = groups % 512;
+  const double rounds = 1.25 * static_cast<double>(groups / 512) + (rest == 0 ? 0.0 : rest <= 256 ? 1.0 : 1.25);
+  return 16.3 + p.bps * rounds * (q6 ? 12.2 : 7.3) + (p.splits > 1 ? 5.4 : 0.0);
 }
 
 SplitActivations SplitForMfma(const float* x, int64_t n_tokens, int64_t cols) {
@@ -1366,17 +1404,12 @@ SplitActivations SplitForMfma(const float* x, int64_t n_tokens, int64_t cols) {
 
 // Launched by GpuMatMulQuantRaw / GpuMatMulQuantGroup for Q4_K / Q6_K with
 // enough tokens; the caller has checked the type, the alignment (Q4_K 16 bytes,
-// Q6_K 2 bytes) and cols % 256 == 0, and split the activations. When the output
-// tiles cannot give every CU a workgroup, K is divided
-// into slices of whole blocks whose partial tiles are summed afterwards in a
-// fixed order (deterministic). Between one and two workgroups per CU the
-// extra pass costs more than the second workgroup slot gains.
+// Q6_K 2 bytes) and cols % 256 == 0, and split the activations.
 void LaunchMatMulMfmaSplit(uint32_t type, const uint8_t* w, int64_t rows, int64_t row_bytes, int32_t nb,
                            const SplitActivations& sa, float* out) {
-  const int64_t gy = (sa.n_tokens + kTileT - 1) / kTileT;
-  const int64_t gx = (rows + kTileR - 1) / kTileR;
-  RPG_CHECK(gy <= 65535 && gx <= 0x7FFFFFFF, "matmul grid too large: %lld x %lld", static_cast<long long>(gx),
-            static_cast<long long>(gy));
+  const GemmPlan plan = PlanGemm(rows, nb, sa.n_tokens);
+  RPG_CHECK(plan.gy <= 65535 && plan.gx <= 0x7FFFFFFF, "matmul grid too large: %lld x %lld",
+            static_cast<long long>(plan.gx), static_cast<long long>(plan.gy));
   RPG_CHECK(static_cast<int64_t>(nb) * kQK_K == sa.cols, "split activations have %lld columns, the matrix %lld",
             static_cast<long long>(sa.cols), static_cast<long long>(nb) * kQK_K);
   // (the planes kernel indexes both operand images with 32-bit offsets;
@@ -1384,7 +1417,7 @@ void LaunchMatMulMfmaSplit(uint32_t type, const uint8_t* w, int64_t rows, int64_
   bool on_planes = kPlanes * sa.n_tokens * sa.cols < (int64_t{1} << 31);
   if (on_planes && sa.n_tokens < kPlanesMinTokens) {
     on_planes = sa.n_tokens >= kPlanesFewTokens &&
-                PlanesUs(type == kGgmlQ6_K, rows, nb, sa.n_tokens) < MfmaUs(rows, nb, sa.n_tokens);
+                PlanesUs(type == kGgmlQ6_K, rows, nb, sa.n_tokens) < MfmaUs(type == kGgmlQ6_K, rows, nb, sa.n_tokens);
   }
   if (on_planes) {
     if (type == kGgmlQ4_K) {
@@ -1395,21 +1428,14 @@ void LaunchMatMulMfmaSplit(uint32_t type, const uint8_t* w, int64_t rows, int64_
     return;
   }
   LaunchPendingSplit(sa);
-  constexpr int64_t kFill = 256;
-  const int64_t tiles = gx * gy;
-  int64_t want = tiles >= kFill ? 1 : (kFill + tiles - 1) / tiles;
-  if (want > nb) want = nb;
-  const int32_t bps = static_cast<int32_t>((nb + want - 1) / want);
-  const int32_t splits = static_cast<int32_t>((nb + bps - 1) / bps);
+  const int32_t splits = plan.splits, bps = plan.bps;
   float* partial = nullptr;
   const int64_t elems = sa.n_tokens * rows;
   if (splits > 1) partial = static_cast<float*>(EnsurePartialTiles(static_cast<size_t>(splits) * elems * sizeof(float)));
-  const dim3 grid(static_cast<unsigned>(gx), static_cast<unsigned>(gy), static_cast<unsigned>(splits));
+  const dim3 grid(static_cast<unsigned>(plan.gx), static_cast<unsigned>(plan.gy), static_cast<unsigned>(splits));
   const _Float16* planes = static_cast<const _Float16*>(sa.planes);
   const _Float16* sums = static_cast<const _Float16*>(sa.sums);
-  // wide matrices (more than 16 row tiles) only while the token tiles are
-  // mostly empty: ffn_gate measured 14% faster at 130 tokens, 9% slower at 256
-  const bool pp = tiles <= kPingPongTiles && (gx <= 16 || sa.n_tokens <= 160);
+  const bool pp = plan.pp;
   const dim3 block(pp ? kGemmThreadsPP : kThreads);
   if (type == kGgmlQ4_K) {
     Launch(pp ? "MatMulMfmaQ4KPingPongKernel" : "MatMulMfmaQ4KKernel",

@@ -737,20 +737,21 @@ __global__ __launch_bounds__(256) void SmallReduceKernel(SmallArgs a, int32_t sl
 
 // Workgroup shapes (waves, half blocks per wave, token tiles) and what they cost:
 // a fixed part (launch, activations, first and last tile) and a part per row tile
-// that a workgroup walks, by weight type: us = fixed + tiles * step. Against MI355X
-// times (graph replay, weights from memory) at 214 sizes of 4 .. 448 tokens on the
-// 1.7B and 4B layer matrices it gives 0.81 to 1.22 of them, nine in ten between 0.84
-// and 1.13: 2048 x 2048 Q4_K at 21 / 448 tokens 7.0 / 24.0 us (measured 7.1 / 27.4),
-// 2048 x 6144 Q6_K at 21 tokens 14.4 (16.2). 16 waves and one token tile are quickest
-// for few tokens and few tiles; two token tiles share a decode and win as the tiles
-// add up; 10 waves fit rows of 10 blocks in two slices.
+// that a workgroup walks, by weight type: us = fixed + tiles * step, fitted to every
+// shape's MI355X times (graph replay, weights from memory) at 1196 sizes of 32 .. 511
+// tokens, 129 .. 32000 rows of 1 .. 56 blocks. From 8 blocks on it gives 0.88 to 1.1 of
+// them (less work per tile is done below), and the shape chosen is within 0.2% of the
+// best: 2048 x 2048 Q4_K at 448 tokens 27 us, 2048 x 6144 Q6_K at 21 tokens 14 (16
+// measured). 16 waves and one token tile are quickest for few tokens and few tiles; two
+// token tiles share a decode and win as the tiles add up; 10 waves fit rows of 10 blocks
+// in two slices.
 struct Shape {
   int w, u, nt;
   double fixed, step4, step6;
 };
-constexpr Shape kShapes[] = {{16, 1, 1, 5.5, 1.55, 1.95}, {8, 2, 2, 8.6, 1.92, 2.55}, {8, 1, 2, 7.0, 1.2, 1.5},
-                             {10, 1, 2, 7.5, 1.5, 2.0}, {10, 2, 1, 7.0, 2.1, 2.9}};
-constexpr double kLoopX = 1.0;  // splitting a slice's activations again for each step
+constexpr Shape kShapes[] = {{16, 1, 1, 4.9, 1.73, 1.83}, {8, 2, 2, 8.2, 2.2, 2.27}, {8, 1, 2, 5.9, 1.36, 1.47},
+                             {10, 1, 2, 7.45, 1.64, 1.76}, {10, 2, 1, 6.4, 2.14, 2.7}};
+constexpr double kLoopX = 1.2;  // splitting a slice's activations again for each step
 constexpr int kShapeCount = sizeof(kShapes) / sizeof(kShapes[0]);
 
 // How a launch of one workgroup shape covers a call: K slices of bps blocks,
@@ -875,8 +876,9 @@ bool MatMulSmallWins(const SmallMat& m, int32_t nb, int64_t n_tokens) {
   // (2048 x 2048 Q4_K: 4.8 us at 2 tokens, 11.4 at 8, against 6.7 here; 2048 x 6144
   // Q6_K: 8.5 and 18.9 against 15).
   if (n_tokens < 32) return us <= 1.1 * (2.4 + (m.q6 ? 0.17 : 0.26) * static_cast<double>(n_tokens) * mega);
-  // The prefill kernels. Within a tenth of them the estimate above is the high one.
-  return us <= 1.1 * std::min(MfmaUs(m.rows, nb, n_tokens), PlanesUs(m.q6, m.rows, nb, n_tokens));
+  // The prefill kernels. (Of the sizes above, 19 take 3 to 7% longer than on those: 2560
+  // x 4864 Q4_K at 320 tokens 61 us and 57.)
+  return us <= std::min(MfmaUs(m.q6, m.rows, nb, n_tokens), PlanesUs(m.q6, m.rows, nb, n_tokens));
 }
 
 void LaunchMatMulSmall(const SmallMat* mats, int32_t n_mats, int32_t nb, const float* x, int64_t n_tokens) {

@@ -40,7 +40,7 @@ void LaunchMatMulMfma(uint32_t type, const uint8_t* w, int64_t rows, int64_t row
 // Estimated times of a prefill matmul: on decoded weight planes (infinite below the
 // tokens that they are used for), and on the GEMM that decodes as it goes.
 double PlanesUs(bool q6, int64_t rows, int32_t nb, int64_t n_tokens);
-double MfmaUs(int64_t rows, int32_t nb, int64_t n_tokens);
+double MfmaUs(bool q6, int64_t rows, int32_t nb, int64_t n_tokens);
 
 // A library-owned buffer of at least `bytes` for the partial results of K slices
 // (valid until the next split launch on the engine stream).

@@ -67,10 +67,11 @@ CASES = [
     ("small batch Q4_K, short prompt", Q4_K, 1024, 2048, 48, "MatMulSmallQ4KKernel"),
     ("matrix cores Q4_K, split K", Q4_K, 9728, 2560, 333,
      "SplitActivationsKernel MatMulMfmaQ4KKernel MatMulSplitReduceKernel"),
-    ("matrix cores Q6_K", Q6_K, 9728, 2560, 400, "SplitActivationsKernel MatMulMfmaQ6KKernel"),
-    ("matrix cores Q6_K, split K, ragged", Q6_K, 4100, 2560, 300,
+    ("matrix cores Q4_K, one block", Q4_K, 19990, 256, 300, "SplitActivationsKernel MatMulMfmaQ4KKernel"),
+    ("matrix cores Q6_K, two blocks", Q6_K, 32000, 512, 200, "SplitActivationsKernel MatMulMfmaQ6KKernel"),
+    ("matrix cores Q6_K, split K, ragged", Q6_K, 9725, 2560, 300,
      "SplitActivationsKernel MatMulMfmaQ6KKernel MatMulSplitReduceKernel"),
-    ("matrix cores Q6_K, two chunks at a time, split K", Q6_K, 9728, 2560, 128,
+    ("matrix cores Q6_K, two chunks at a time, split K", Q6_K, 16380, 2560, 128,
      "SplitActivationsKernel MatMulMfmaQ6KPingPongKernel MatMulSplitReduceKernel"),
     ("matrix cores Q4_K, two chunks at a time, split K", Q4_K, 13808, 4352, 110,
      "SplitActivationsKernel MatMulMfmaQ4KPingPongKernel MatMulSplitReduceKernel"),

@@ -45,11 +45,10 @@ gen = torch.Generator(device="cuda")
 gen.manual_seed(1)
 
 
-def matrix(t, rows):
-    nb, bb = rows * 10, ops.BLOCK_BYTES[t]
-    b = torch.randint(0, 256, (nb, bb), generator=gen, device="cuda", dtype=torch.uint8)
-    b[:, slice(0, 4) if t == 12 else slice(208, 210)] = 20  # the fp16 scales: 0x1414
-    return ops.GpuTensor(b.reshape(-1), t, rows, 2560)
+def matrix(rows, cols):
+    b = torch.randint(0, 256, (rows * cols // 256, 144), generator=gen, device="cuda", dtype=torch.uint8)
+    b[:, 0:4] = 20  # the fp16 scales: 0x1414
+    return ops.GpuTensor(b.reshape(-1), 12, rows, cols)
 
 
 def capture(w, x, out, refused):
@@ -75,12 +74,12 @@ def kernels(call):
     return set(ops.profile_report())
 
 
-w, other = matrix(12, 9728), matrix(14, 9728)
+w, other = matrix(9728, 2560), matrix(9728, 3072)
 x = torch.randn(448, 2560, generator=gen, device="cuda")
 out, eager = (torch.empty(448, 9728, device="cuda") for _ in range(2))
 # the activations' buffer, from a call on the GEMM that decodes as it goes
-assert "MatMulMfmaQ6KKernel" in kernels(lambda: ops.GpuMatMulQuant(other, x[:385], 385, eager))
-assert "MatMulMfmaQ6KKernel" in kernels(lambda: ops.GpuMatMulQuant(other, x, 448, eager))
+x3 = torch.randn(384, 3072, generator=gen, device="cuda")
+assert "MatMulMfmaQ4KKernel" in kernels(lambda: ops.GpuMatMulQuant(other, x3, 384, eager))
 capture(w, x, out, True)
 assert "MatMulMfmaQ4KPlanesKernel" in kernels(lambda: ops.GpuMatMulQuant(w, x, 448, eager))
 graph = capture(w, x, out, False)

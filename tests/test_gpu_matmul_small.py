@@ -193,3 +193,19 @@ def test_group_refuses_null_activations(gpu, n):
     outs = [torch.empty((n, 2048), device="cuda") for _ in ws]
     with pytest.raises(gpu.RpgError, match="null pointer"):
         gpu.GpuMatMulQuantGroup(ws, None, n, outs)
+
+
+@pytest.mark.parametrize("t,rows,cols,n,kernel", [
+    # measured there and here, us: 74 and 103, 84 and 120, 94 and 106, 99 and 108; 12.4 and 14.3
+    (Q4, 9728, 2560, 300, "MatMulMfmaQ4KKernel"), (Q4, 5120, 5120, 333, "MatMulMfmaQ4KKernel"),
+    (Q4, 2560, 9728, 333, "MatMulMfmaQ4KKernel"), (Q6, 9728, 2560, 300, "MatMulMfmaQ6KKernel"),
+    (Q4, 2048, 6144, 3, "MatMulQ4KKernel"),
+    # 55 and 43, 123 and 104, 141 and 128, 36 and 22
+    (Q4, 6144, 2048, 300, "MatMulSmallQ4KKernel"), (Q6, 2560, 9728, 333, "MatMulSmallQ6KKernel"),
+    (Q6, 32000, 2048, 200, "MatMulSmallQ6KKernel"), (Q4, 6144, 2048, 128, "MatMulSmallQ4KKernel")])
+def test_small_route_is_the_faster_kernel(gpu, t, rows, cols, n, kernel):
+    import torch
+
+    w = torch.zeros(rows * cols // 256 * (144 if t == Q4 else 210), dtype=torch.uint8, device="cuda")
+    x, out = torch.zeros((n, cols), device="cuda"), torch.empty((n, rows), device="cuda")
+    assert kernel in launches(gpu, lambda: gpu.GpuMatMulQuant(gpu.GpuTensor(w, t, rows, cols), x, n, out))
