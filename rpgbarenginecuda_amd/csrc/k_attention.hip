@@ -1183,7 +1183,10 @@ __global__ __launch_bounds__(256, 2) void AttnPrefillMfmaKernel(
   const int64_t pos0 = ReadPos0(pos0_val, pos0_dev);
   const int64_t tq = t0 + 32 * wv + col;
   const bool qvalid = tq < seq;
-  const int64_t qpos = pos0 + tq;
+  // The last key that token t sees. (The cache's end comes first only in a replayed graph
+  // with a bad staged pos0.)
+  const auto sees = [&](int64_t t) { return pos0 + t < max_seq ? pos0 + t : max_seq - 1; };
+  const int64_t qpos = sees(tq);
 
   F16x8 qb[2][8];
   float sinv;
@@ -1195,9 +1198,9 @@ __global__ __launch_bounds__(256, 2) void AttnPrefillMfmaKernel(
   float m = -INFINITY, l = 0.0f;
 
   const int64_t t_last = (t0 + kFaTokens < seq ? t0 + kFaTokens : seq) - 1;
-  const int64_t last_key = pos0 + t_last;                                   // the workgroup's causal limit
-  const int64_t wave_last = pos0 + (t0 + 32 * wv + 31 < seq ? t0 + 32 * wv + 31 : seq - 1);
-  const int64_t wave_first = pos0 + t0 + 32 * wv;   // the wave's first query position
+  const int64_t last_key = sees(t_last);            // the workgroup's causal limit
+  const int64_t wave_last = sees(t0 + 32 * wv + 31 < seq ? t0 + 32 * wv + 31 : seq - 1);
+  const int64_t wave_first = sees(t0 + 32 * wv);    // the wave's first query position
   const bool wave_full = t0 + 32 * wv + 31 < seq;   // all 32 queries of the wave are tokens
   const uint16_t* kbase = kc + static_cast<int64_t>(kh) * max_seq * kD;
   const uint16_t* vbase = vc + static_cast<int64_t>(kh) * max_seq * kD;
@@ -1490,8 +1493,7 @@ __global__ __launch_bounds__(64 * kTurnWaves, 1) void AttnTurnKernel(
   const bool qvalid = tq < seq;
   const int64_t pos0 = ReadPos0(pos0_val, pos0_dev);
   const bool full = t_first + kTurnRows <= seq;
-  // The last keys that the tile's first token, this lane's and the tile's last one see. (The
-  // cache's end comes first only in a replayed graph with a bad staged pos0.)
+  // as in AttnPrefillMfmaKernel, for the tile's first token, this lane's and the tile's last
   const auto sees = [&](int64_t t) { return pos0 + t < max_seq ? pos0 + t : max_seq - 1; };
   const int64_t first_key = sees(t_first), my_key = sees(tq), last_key = sees((full ? t_first + kTurnRows : seq) - 1);
 

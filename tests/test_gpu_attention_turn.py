@@ -134,17 +134,19 @@ def test_prefill_unaligned_values(gpu, seq):
     assert torch.equal(*outs)
 
 
-def test_turn_staged_past_the_cache(gpu, ora):
-    """A replay whose staged position puts tokens past the cache's end: they see the whole
+@pytest.mark.parametrize("max_seq,seq", [(2048, 45), (2048, 64), (700, 200), (4001, 300)])
+def test_staged_past_the_cache(gpu, ora, max_seq, seq):
+    """A turn or a prefill: a replay whose staged position puts tokens past the cache's end: they see the whole
     cache, and nothing behind it is read (as the decode kernel does)."""
     import torch
 
-    nh, nkv, max_seq, seq = 16, 8, 2048, 45
-    rng = np.random.default_rng(12)
+    nh, nkv = 16, 8
+    rng = np.random.default_rng(max_seq + seq)
     q, kc, vc = make(rng, nh, nkv, max_seq, seq, qscale=0.5)
     qd, kd, vd = dev(q), dev(kc), dev(vc)
     out = torch.empty((seq, nh, 128), dtype=torch.float32, device="cuda")
     gpu.init()
+    gpu.GpuAttentionFromCache(nh, nkv, 128, 0, qd, seq, kd, vd, max_seq, out, max_seq)  # the library's buffers
     stream = torch.cuda.Stream()
     stream.wait_stream(torch.cuda.current_stream())
     graph = torch.cuda.CUDAGraph()
@@ -161,7 +163,7 @@ def test_turn_staged_past_the_cache(gpu, ora):
         graph.replay()
         torch.cuda.synchronize()
         got = host(out)
-        for t in (0, 19, 20, 33, 44):
+        for t in (0, 19, 20, 33, seq - 1):
             at = min(pos + t, max_seq - 1)
             ref, smag, vmax = ora.attention_f64(q[t:t + 1], kc, vc, max_seq, nh, nkv, 128, at, 1)
             check(got[t:t + 1], ref, smag, vmax, at)
