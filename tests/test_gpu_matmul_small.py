@@ -1,13 +1,14 @@
 """The small-batch quantised matmul (2 tokens to a medium prompt): every workgroup shape
 at the edges of its tiles, against the float64 oracle within the fp32 summation
-bound of tests/test_gpu_matmul.py, and against itself where the bits must agree."""
+bound of tests/test_gpu_matmul.py, and against itself where the bits must agree. The
+sizes are ones that the rule sends to the kernel; each test checks that it ran."""
 from __future__ import annotations
 
 import numpy as np
 import pytest
 
 import synth
-from test_gpu_matmul import check, dev, factored_magnitude, host
+from test_gpu_matmul import check, dev, host
 
 pytestmark = pytest.mark.gpu
 
@@ -20,16 +21,40 @@ def launches(gpu, call):
     return set(gpu.profile_report())
 
 
+def small(gpu, t, call):
+    """The call's launches are the kernel of that type, and perhaps its reduce."""
+    return launches(gpu, call) - {"MatMulSmallReduceKernel"} == {"MatMulSmallQ%dKKernel" % (4 if t == Q4 else 6)}
+
+
+def centred_magnitude(ora, t, w, rows, cols, x):
+    """Q4_K only: sum_e (|d1 (q_e - 8)| + |8 d1 - m1|) |x_e|, the terms that the kernel sums:
+    it multiplies by the centred quants and adds what the centring took by the runs' sums.
+    (A column a thousand times the others with quant 0 and a small m1 rounds by 8 d1 of it,
+    which the weight itself does not bound.) A copy of the matrix with every quant 8
+    dequantises to 8 d1 - m1."""
+    if t != Q4:
+        return 0.0
+    z = np.array(w, copy=True).reshape(-1, 144)
+    z[:, 16:] = 0x88
+    n = rows * cols
+    wd = ora.dequantize_row(t, np.ascontiguousarray(w), n).reshape(rows, cols).astype(np.float64)
+    w8 = ora.dequantize_row(t, z.reshape(-1), n).reshape(rows, cols).astype(np.float64)
+    return np.abs(np.asarray(x, np.float64).reshape(-1, cols)) @ (np.abs(wd - w8) + np.abs(w8)).T
+
+
 SHAPES = [
     # (type, rows, cols, tokens)
-    (Q4, 1, 256, 5), (Q6, 1, 256, 6),            # one row, one block
-    (Q4, 17, 768, 16), (Q6, 15, 768, 17),        # ragged row tile, odd blocks, one token over a tile
-    (Q6, 300, 2048, 31), (Q4, 300, 2048, 33),    # both sides of the slices' limit
-    (Q4, 2049, 2048, 65), (Q6, 2049, 2048, 97),  # ragged rows and token tiles, several tiles per workgroup
-    (Q4, 65, 2304, 9), (Q6, 65, 2560, 10),       # 9 and 10 blocks
-    (Q4, 1000, 2816, 8), (Q6, 1000, 2816, 40),   # 11 blocks: walked by a workgroup, in slices of unequal length
-    (Q6, 500, 9728, 30), (Q4, 500, 9728, 36),    # 38 blocks likewise
-    (Q6, 20000, 2048, 17), (Q4, 20000, 512, 21),  # many tiles
+    (Q4, 1, 256, 33), (Q6, 1, 256, 40),            # one row, one block
+    (Q4, 17, 768, 36), (Q6, 15, 768, 49),          # ragged row tile, odd blocks, one token over a tile
+    (Q4, 2049, 2048, 9), (Q4, 700, 2048, 31), (Q4, 300, 2048, 33),  # up to the slices' limit and over it
+    (Q6, 7001, 1280, 25),                          # 5 blocks: waves with nothing to do
+    (Q4, 2049, 2048, 65), (Q6, 2049, 2048, 97),    # ragged rows and token tiles, several tiles per workgroup
+    (Q6, 20001, 2048, 17), (Q4, 20000, 512, 21),   # many tiles
+    (Q4, 9001, 768, 16), (Q6, 9003, 512, 21), (Q4, 30001, 256, 9),  # short rows
+    (Q6, 3003, 2304, 10), (Q4, 3001, 2560, 19),    # 9 and 10 blocks
+    (Q6, 5001, 2560, 100), (Q4, 5001, 2560, 150),  # 10 blocks in two slices
+    (Q6, 2001, 2816, 30), (Q6, 1000, 2816, 40),    # 11 blocks: walked by a workgroup, in slices of unequal length
+    (Q4, 2501, 9728, 18), (Q6, 500, 9728, 30), (Q4, 500, 9728, 36),  # 38 blocks likewise
 ]
 
 
@@ -43,26 +68,26 @@ def test_small_matmul_vs_f64(gpu, ora, t, rows, cols, n):
     x[n // 2] *= 1e-20  # tokens of very different size keep their own scale
     x[:, cols // 2] *= 1e3
     out = torch.full((n + 1, rows), np.nan, dtype=torch.float32, device="cuda")
-    gpu.GpuMatMulQuant(gpu.GpuTensor(dev(w), t, rows, cols), dev(x), n, out[:n])
+    assert small(gpu, t, lambda: gpu.GpuMatMulQuant(gpu.GpuTensor(dev(w), t, rows, cols), dev(x), n, out[:n]))
     exact, absdot = ora.matmul_quant_f64(t, w, rows, cols, x)
-    check(host(out[:n]), exact, absdot, cols, factored_magnitude(ora, t, w, rows, cols, x))
+    check(host(out[:n]), exact, absdot, cols, centred_magnitude(ora, t, w, rows, cols, x))
     assert torch.isnan(out[n]).all(), "wrote past the last token"
 
 
 @pytest.mark.parametrize("off", [2, 6, 14])
-def test_small_matmul_unaligned_q6k(gpu, off):
+@pytest.mark.parametrize("rows,cols,n", [(2501, 2560, 21), (2001, 2816, 30), (131, 2560, 40)])
+def test_small_matmul_unaligned_q6k(gpu, rows, cols, n, off):
     """A Q6_K matrix at any even address gives the bits of the aligned one."""
     import torch
 
-    rows, cols, n = 130, 2560, 21
     rng = np.random.default_rng(off)
     w = dev(synth.quant_table(rng, Q6, rows, cols))
     moved = torch.zeros(w.numel() + 64, dtype=torch.uint8, device="cuda")
     moved[off:off + w.numel()] = w
     x = dev(rng.normal(0, 1, (n, cols)).astype(np.float32))
     outs = [torch.empty((n, rows), device="cuda") for _ in range(2)]
-    gpu.GpuMatMulQuant(gpu.GpuTensor(w, Q6, rows, cols), x, n, outs[0])
-    gpu.GpuMatMulQuant(gpu.GpuTensor(moved[off:off + w.numel()], Q6, rows, cols), x, n, outs[1])
+    for buf, out in zip((w, moved[off:off + w.numel()]), outs):
+        assert small(gpu, Q6, lambda: gpu.GpuMatMulQuant(gpu.GpuTensor(buf, Q6, rows, cols), x, n, out))
     assert torch.equal(*outs)
 
 
@@ -91,19 +116,18 @@ def test_small_group_and_swiglu_equal_separate_calls(gpu, cols, n):
 
 
 @pytest.mark.parametrize("t", [Q4, Q6])
-@pytest.mark.parametrize("cols,n", [(2048, 40), (6144, 24), (6144, 48)])
-def test_small_one_hot_selects_columns(gpu, ora, t, cols, n):
+@pytest.mark.parametrize("rows,cols,n", [(40, 2048, 40), (1500, 6144, 24), (40, 6144, 48)])
+def test_small_one_hot_selects_columns(gpu, ora, t, rows, cols, n):
     """A single activation 1 gives the dequantised weight, bit for bit."""
     import torch
 
-    rows = 40
     rng = np.random.default_rng(t + cols + n)
     w = synth.quant_table(rng, t, rows, cols)
     picks = rng.permutation(cols)[:n]
     x = np.zeros((n, cols), np.float32)
     x[np.arange(n), picks] = 1.0
     out = torch.empty((n, rows), device="cuda")
-    gpu.GpuMatMulQuant(gpu.GpuTensor(dev(w), t, rows, cols), dev(x), n, out)
+    assert small(gpu, t, lambda: gpu.GpuMatMulQuant(gpu.GpuTensor(dev(w), t, rows, cols), dev(x), n, out))
     want = ora.dequantize_row(t, w, rows * cols).reshape(rows, cols)[:, picks].T
     assert np.array_equal(host(out), want)
 
@@ -112,7 +136,7 @@ def test_small_matmul_captures_without_a_first_run(gpu):
     """Below 32 tokens a call needs no buffer of the library, also for a long K."""
     import torch
 
-    rows, cols, n = 64, 16384, 7
+    rows, cols, n = 3000, 16384, 7
     rng = np.random.default_rng(5)
     w = gpu.GpuTensor(dev(synth.quant_table(rng, Q4, rows, cols)), Q4, rows, cols)
     x = dev(rng.normal(0, 1, (n, cols)).astype(np.float32))
@@ -125,7 +149,7 @@ def test_small_matmul_captures_without_a_first_run(gpu):
         x *= scale
         out.fill_(float("nan"))
         g.replay()
-        gpu.GpuMatMulQuant(w, x, n, eager)
+        assert launches(gpu, lambda: gpu.GpuMatMulQuant(w, x, n, eager)) == {"MatMulSmallQ4KKernel"}
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
 
@@ -151,7 +175,7 @@ def test_small_infinite_activation(gpu, ora, t, rows, cols, n):
     x[bad[2], 0] = np.nan
     xd = dev(x)
     outs = [torch.empty((n, rows), device="cuda") for _ in range(3)]
-    gpu.GpuMatMulQuant(ws[0], xd, n, outs[0])
+    assert small(gpu, t, lambda: gpu.GpuMatMulQuant(ws[0], xd, n, outs[0]))
     gpu.GpuMatMulQuantGroup(ws, xd, n, outs[1:])
     gate, up = torch.empty((n, rows), device="cuda"), torch.empty((n, rows), device="cuda")
     gpu.GpuMatMulQuantSwiGLU(ws[0], ws[1], xd, n, gate, up)
