@@ -1,7 +1,6 @@
 """The matmul on decoded weight planes (512 tokens and more, and fewer on large
-matrices): ragged row groups, row and
-token tiles, one block to several, against the float64 oracle within the bound of
-tests/test_gpu_matmul.py."""
+matrices): ragged row groups, row and token tiles, one block to several, against the
+float64 oracle within the bound of tests/test_gpu_matmul.py."""
 from __future__ import annotations
 
 import os
@@ -30,7 +29,10 @@ def test_planes_matmul_vs_f64(gpu, ora, t, rows, cols, n):
     x = rng.normal(0, 1, (n, cols)).astype(np.float32)
     x[n // 2] *= 1e-20  # tokens of very different size keep their own scale
     out = torch.full((n + 1, rows), np.nan, dtype=torch.float32, device="cuda")
+    gpu.profile_start(16)
     gpu.GpuMatMulQuant(gpu.GpuTensor(dev(w), t, rows, cols), dev(x), n, out[:n])
+    gpu.profile_stop()
+    assert "MatMulMfmaQ%dKPlanesKernel" % (4 if t == Q4 else 6) in gpu.profile_report()
     exact, absdot = ora.matmul_quant_f64(t, w, rows, cols, x)
     check(host(out[:n]), exact, absdot, cols, factored_magnitude(ora, t, w, rows, cols, x))
     assert torch.isnan(out[n]).all(), "wrote past the last token"
