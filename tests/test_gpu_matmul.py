@@ -95,15 +95,19 @@ SHAPES = [
     (12, 777, 2048, 8),
     (14, 513, 2048, 13),     # two tiles of 8, the second ragged
     (12, 256, 256, 21),      # the CPU-runnable n = 21
-    (12, 2048, 2048, 64),    # matrix-core GEMM: one token tile, 16 row tiles
+    (12, 2048, 2048, 64),    # small-batch kernel
     (14, 1024, 2048, 130),   # ragged token tiles
     (12, 300, 2560, 200),    # ragged row tile, 10 blocks per row
-    (14, 777, 6144, 129),    # 24 blocks per row, ragged both ways
-    (14, 128, 256, 32),      # the smallest matrix-core case
-    (12, 64, 512, 31),       # just below it: the tiled kernel
-    (12, 6144, 2048, 17),    # wide matrix: matrix cores from 16 tokens, K split 8 ways
-    (14, 4096, 2560, 16),    # ... Q6_K, 10 blocks per row split one each
-    (12, 4095, 2048, 16),    # one row short of wide: the tiled kernel
+    (14, 777, 6144, 129),    # 24 blocks per row, ragged both ways, K slices
+    (14, 128, 256, 32),      # one block per row
+    (12, 64, 512, 31),       # few rows and fewer tokens: the tiled kernel
+    (12, 6144, 2048, 17),    # small-batch kernel, several tiles per workgroup
+    (14, 4096, 2560, 16),    # ... Q6_K, 10 blocks per row
+    (12, 4095, 2048, 16),    # ... ragged row tile
+    (12, 19990, 256, 300),   # GEMM decoding as it goes: ragged row and token tiles, one block per row
+    (12, 32000, 512, 100),   # ... K split
+    (14, 31999, 512, 100),   # ... Q6_K
+    (12, 14001, 768, 300),   # ... 3 blocks per row, no split
     (12, 2048, 2048, 600),   # decoded weight planes (from 512 tokens): 8 x 5 tiles, K split
     (14, 1024, 2048, 700),   # ... Q6_K, ragged token tile, K split
     (12, 1100, 2560, 513),   # ... ragged row tile (1100 = 4.3 x 256), 10 blocks per row
@@ -185,8 +189,12 @@ def test_matmul_q6k_extreme_scales(gpu, ora):
     summation bound, and -128 * -32 * d exact."""
     import torch
 
-    cols = 2048
-    for rows, n in ((16400, 1), (1024, 1), (300, 5), (2048, 64)):
+    # one token (two kernels), the tiled one, small batches without and with K slices in a
+    # workgroup, the GEMM that decodes as it goes, its two-chunk form, the weight planes
+    for rows, cols, n, kernel in ((16400, 2048, 1, "MatVecQ6K"), (2048, 6144, 1, "MatVecSplitQ6K"), (300, 2048, 5, "MatMulQ6K"),
+                                  (2048, 2048, 64, "MatMulSmallQ6K"), (2048, 6144, 21, "MatMulSmallQ6K"),
+                                  (31999, 512, 100, "MatMulMfmaQ6KK"), (16380, 2560, 100, "MatMulMfmaQ6KPingPong"),
+                                  (300, 2048, 600, "MatMulMfmaQ6KPlanes")):
         case(f"matmul Q6_K extreme scales [{rows} x {cols}] x {n}")
         rng = np.random.default_rng(792 + n)
         w = synth.quant_table(rng, 14, rows, cols).reshape(-1, 210)
@@ -197,7 +205,10 @@ def test_matmul_q6k_extreme_scales(gpu, ora):
         w = w.reshape(-1)
         x = rng.normal(0, 1, (n, cols)).astype(np.float32)
         out = torch.full((n, rows), np.nan, dtype=torch.float32, device="cuda")
+        gpu.profile_start(16)
         gpu.GpuMatMulQuant(gpu.GpuTensor(dev(w), 14, rows, cols), dev(x), n, out)
+        gpu.profile_stop()
+        assert any(k.startswith(kernel) for k in gpu.profile_report()), kernel
         exact, absdot = ora.matmul_quant_f64(14, w, rows, cols, x)
         check(host(out), exact, absdot, cols)
 
