@@ -19,7 +19,8 @@
 //   * Q4_K weights enter centred, sc_j (q - 8), an exact fp16 integer: the partial
 //     sums are half of those of sc_j q, and so is their rounding. The rest, (8 d sc_j -
 //     dmin m_j) times the sub-block's sum of x, comes from one double-precision
-//     matrix product per half block and joins in double;
+//     matrix product per half block and joins in double. (A column far larger than the
+//     others whose quant is near 0 is the other way round: it rounds by 8 d sc_j of it.)
 //   * Q6_K weights enter as w = sc (q - 32) in two exact fp16 terms (w rounded, and
 //     the remainder, nonzero only for |w| > 2048); the matrix cores form x_hi w_hi,
 //     x_lo w_hi and x_hi w_lo; x_lo w_lo is below 2^-22 |x w|.
@@ -28,9 +29,9 @@
 //
 // Measured on MI355X (graph replay, weights rotated past the Infinity Cache), against
 // the tiled kernel (below 16 or 32 tokens) and the prefill GEMM that ran these sizes:
-// q / k / v of a 1.7B layer, 21 tokens 46.6 -> 9.2 us, 128 tokens 69.8 -> 18.3; gate / up
-// with SwiGLU 43.6 -> 17.3 and 71.6 -> 34.2; ffn_down 40.8 -> 18.7 and 39.8 -> 29.7;
-// the 151936-row output projection at 21 tokens 350 -> 118. What a tile of 16 rows costs
+// q / k / v of a 1.7B layer, 21 tokens 46.6 -> 9.4 us, 128 tokens 69.8 -> 19.0; gate / up
+// with SwiGLU 43.6 -> 17.8 and 71.6 -> 36.7; ffn_down 40.8 -> 16.9 and 39.8 -> 28.5;
+// the 151936-row output projection at 21 tokens 350 -> 104. What a tile of 16 rows costs
 // now is mostly its ~130 vector instructions per wave and half block, of which the
 // decode is 40; loading x in the matrix core's own layout (4 us more per call: one cache
 // line per lane instead of one per four) and the weights one lane's bytes at a time
@@ -785,7 +786,10 @@ double ShapeCost(int shape, int nb, int64_t n_tokens, int64_t rows, bool q6) {
   const Plan p = PlanFor(shape, nb, n_tokens, static_cast<int>((rows + 15) / 16));
   if (p.loops > 1 && shape != 0) return 1e9;  // built for the first shape only
   const double reduce = p.slices > 1 ? 2.2 + 8.0 * p.slices * static_cast<double>(n_tokens) * static_cast<double>(rows) / 5e6 : 0.0;
-  const double step = (q6 ? s.step6 : s.step4) + (p.loops > 1 ? kLoopX : 0.0);
+  // rows of 1 to 3 blocks leave waves without work (12000 x 512 Q4_K, 224 tokens: 26 us
+  // on the third shape, 37 on the second; 35 on the GEMM)
+  const double share = nb < 4 ? 0.5 + nb / static_cast<double>(s.w * s.u) : 1.0;
+  const double step = share * (q6 ? s.step6 : s.step4) + (p.loops > 1 ? kLoopX : 0.0);
   return s.fixed + p.iters * p.loops * step + reduce;
 }
 
@@ -876,8 +880,8 @@ bool MatMulSmallWins(const SmallMat& m, int32_t nb, int64_t n_tokens) {
   // (2048 x 2048 Q4_K: 4.8 us at 2 tokens, 11.4 at 8, against 6.7 here; 2048 x 6144
   // Q6_K: 8.5 and 18.9 against 15).
   if (n_tokens < 32) return us <= 1.1 * (2.4 + (m.q6 ? 0.17 : 0.26) * static_cast<double>(n_tokens) * mega);
-  // The prefill kernels. (Of the sizes above, 19 take 3 to 7% longer than on those: 2560
-  // x 4864 Q4_K at 320 tokens 61 us and 57.)
+  // The prefill kernels. (Of 2288 sizes of 2 to 511 tokens, 13 take 3 to 9% longer than on
+  // the fastest kernel, all with Q4_K of few rows: 2560 x 4864 at 320 tokens 61 us and 57.)
   return us <= std::min(MfmaUs(m.q6, m.rows, nb, n_tokens), PlanesUs(m.q6, m.rows, nb, n_tokens));
 }
 

@@ -224,9 +224,10 @@ def test_group_refuses_null_activations(gpu, n):
     (Q4, 9728, 2560, 300, "MatMulMfmaQ4KKernel"), (Q4, 5120, 5120, 333, "MatMulMfmaQ4KKernel"),
     (Q4, 2560, 9728, 333, "MatMulMfmaQ4KKernel"), (Q6, 9728, 2560, 300, "MatMulMfmaQ6KKernel"),
     (Q4, 2048, 6144, 3, "MatMulQ4KKernel"),
-    # 55 and 43, 123 and 104, 141 and 128, 36 and 22
+    # 55 and 43, 123 and 104, 141 and 128, 36 and 22, 35 and 26
     (Q4, 6144, 2048, 300, "MatMulSmallQ4KKernel"), (Q6, 2560, 9728, 333, "MatMulSmallQ6KKernel"),
-    (Q6, 32000, 2048, 200, "MatMulSmallQ6KKernel"), (Q4, 6144, 2048, 128, "MatMulSmallQ4KKernel")])
+    (Q6, 32000, 2048, 200, "MatMulSmallQ6KKernel"), (Q4, 6144, 2048, 128, "MatMulSmallQ4KKernel"),
+    (Q4, 12000, 512, 224, "MatMulSmallQ4KKernel")])
 def test_small_route_is_the_faster_kernel(gpu, t, rows, cols, n, kernel):
     import torch
 
