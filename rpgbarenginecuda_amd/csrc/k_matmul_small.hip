@@ -881,7 +881,8 @@ bool MatMulSmallWins(const SmallMat& m, int32_t nb, int64_t n_tokens) {
   // Q6_K: 8.5 and 18.9 against 15).
   if (n_tokens < 32) return us <= 1.1 * (2.4 + (m.q6 ? 0.17 : 0.26) * static_cast<double>(n_tokens) * mega);
   // The prefill kernels. (Of 2288 sizes of 2 to 511 tokens, 13 take 3 to 9% longer than on
-  // the fastest kernel, all with Q4_K of few rows: 2560 x 4864 at 320 tokens 61 us and 57.)
+  // the GEMM: 5120 x 5120 Q6_K at 333 tokens 123 us and 113, 2560 x 9728 Q4_K at 256 78
+  // and 74.)
   return us <= std::min(MfmaUs(m.q6, m.rows, nb, n_tokens), PlanesUs(m.q6, m.rows, nb, n_tokens));
 }
 
