@@ -91,7 +91,7 @@ def test_small_matmul_unaligned_q6k(gpu, rows, cols, n, off):
     assert torch.equal(*outs)
 
 
-@pytest.mark.parametrize("cols,n", [(2048, 21), (2048, 40), (2048, 200), (2560, 21), (2560, 70), (6144, 20), (6144, 50)])
+@pytest.mark.parametrize("cols,n", [(256, 30), (512, 100), (768, 40), (2048, 21), (2048, 40), (2048, 200), (2560, 21), (2560, 70), (6144, 20), (6144, 50)])
 def test_small_group_and_swiglu_equal_separate_calls(gpu, cols, n):
     """Matrices of both types and of sizes that prefer different shapes, each bit-identical to its own call;
     gate / up likewise to the two products followed by SwiGLU."""
