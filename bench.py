@@ -1049,7 +1049,7 @@ def host_cpu():
 
 
 # CPU threads of the baseline: every thread the process may use, capped at the
-# 16-thread CPU share a one-GPU job gets on the GPU boxes (the host itself can
+# 16-thread CPU share a one-GPU job gets on the machines measured (the host itself can
 # have many more logical CPUs; both counts are reported).
 CPU_SHARE = 16
 

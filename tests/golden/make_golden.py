@@ -7,7 +7,7 @@ The reference's src/quant.cc + src/common.cc are compiled where they lie into
 oracle/_ref/libref_quant.so (oracle/Makefile); this script feeds them seeded
 synthetic Q4_K / Q6_K blocks (plus hand-made edge-case blocks) and stores inputs
 and outputs. The fixture is data only: raw block bytes in, fp32 bit patterns out.
-It lets tests on the GPU box, where the reference does not exist, check the
+It lets tests on a GPU machine, where the reference does not exist, check the
 oracle and the device path against the reference's own answers.
 
 Also stored: the reference F16ToF32 over all 65536 halves (as a SHA-256 of the
